@@ -50,6 +50,7 @@ constexpr int kShadeBlock = 256;
 #define BB_RESERVOIR 128
 #endif
 constexpr int kReservoir = BB_RESERVOIR; // queries a traversal wave claims per atomic
+constexpr int kFirstChunkMin = 8; // fewest queries a wave starts with
 constexpr int kLdsCdfEntries = 2049; // lights whose CDF the shading kernel keeps in LDS (up to 2048)
 constexpr int kMaxGridBlocks = 256 * 32;
 
@@ -509,10 +510,28 @@ BB_D bool trace_step(const SceneView& S, Lane& L, const TraceStack<StackEntry<AN
     return false;
 }
 
-// Persistent traversal: a wave takes consecutive queries from the shared
-// counter `fetch` and hands a new query to its idle lanes once at least
-// `refill_min` of its 64 lanes are idle (64: whole-wave batches, one atomic
-// per 64 queries).  Between refill checks every lane takes STEPS traversal
+// Queries a wave takes before the shared counter: its own part of [0, n),
+// `chunk` of them, found without an atomic; the counter serves what lies
+// beyond waves * chunk.  When every wave asked the counter first, the
+// same-address atomics of the 7,168 waves of a full grid cost 84 us even for
+// an empty queue (two launches per depth: 1.5 of the 2.3 ms of the README
+// frame at 640 x 360 x 16 spp; 0.82 ms now).  The even split also spreads a
+// short queue over the whole chip instead of filling few waves 128 deep,
+// whose rays then ran one refill after another: a 1280 x 720 frame of 1 spp
+// (82 K triangles) takes 2.77 instead of 4.69 ms.  Fewer than 8 queries a
+// wave gain nothing more there (1: 2.86, 4: 2.80, 8: 2.77, 16: 2.77, 64:
+// 2.89 ms); a batch of 61 rays alone would take 60 us with 1, 64 with 8, 69
+// with 64.
+BB_HD int first_chunk(int n, int waves)
+{
+    const int even = n / waves + (n % waves != 0 ? 1 : 0);
+    return even < kFirstChunkMin ? kFirstChunkMin : (even > kReservoir ? kReservoir : even);
+}
+
+// Persistent traversal: a wave starts with its own part of the queries
+// (first_chunk), then takes consecutive ones from the shared counter `fetch`,
+// and hands a new query to its idle lanes once at least `refill_min` of its
+// 64 lanes are idle.  Between refill checks every lane takes STEPS traversal
 // steps.  Src provides load(index, Lane&) and finish(index, const Lane&).
 template <bool ANY, bool COUNT, int SK, bool ALPHA, int STEPS, typename Src>
 BB_D void persistent_trace(const SceneView& S, const Src& src, int n, int* fetch,
@@ -521,22 +540,25 @@ BB_D void persistent_trace(const SceneView& S, const Src& src, int n, int* fetch
     const int lane = __lane_id();
     const unsigned long long below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
     Lane L;
-    bool active = false, more = true;
+    bool active = false;
     int id = 0;
-    // the wave's reservoir of claimed queries [rb, re): claimed kReservoir
-    // at a time, so the shared counter sees one atomic per kReservoir
-    // queries instead of one per refill (same-address atomics limit the rate)
-    int rb = 0, re = 0;
+    // the wave's reservoir of claimed queries [rb, re)
+    const int waves = gridDim.x * (blockDim.x >> 6);
+    const int wave = __builtin_amdgcn_readfirstlane(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6));
+    const int chunk = first_chunk(n, waves);
+    const int shared = waves * chunk; // queries from here on are claimed from the counter
+    int rb = min(wave * chunk, n), re = min(wave * chunk + chunk, n);
+    bool more = shared < n;
     for (;;) {
         unsigned long long idle = __ballot(active ? 0 : 1);
         if ((more || rb < re) && (__popcll(idle) >= refill_min || idle == ~0ull)) {
             if (rb >= re) {
                 int base = 0;
                 if (lane == 0) base = atomicAdd(fetch, kReservoir);
-                base = __shfl(base, 0);
-                rb = base;
-                re = base + kReservoir < n ? base + kReservoir : n;
-                if (base + kReservoir >= n) more = false;
+                const unsigned b = unsigned(shared) + unsigned(__shfl(base, 0)); // below 2^31 + waves * kReservoir
+                rb = b < unsigned(n) ? int(b) : n;
+                re = n - rb > kReservoir ? rb + kReservoir : n;
+                if (re == n) more = false;
             }
             const int rank = __popcll(idle & below);
             const int mine = rb + rank;
@@ -1775,6 +1797,9 @@ size_t trace_lds_bytes(int lds_entries, bool slim = false, int block = kTraceBlo
     return size_t(lds_entries) * size_t(block) * (slim ? sizeof(int) : sizeof(int2));
 }
 
+// blocks that n queries can keep busy, kFirstChunkMin queries per wave
+int trace_blocks(long long n, int block) { return grid_for(n, (block / 64) * kFirstChunkMin); }
+
 // persistent grid of a traversal kernel: resident blocks per CU x CUs
 int trace_grid(const void* kernel, size_t lds_bytes, int block = kTraceBlock)
 {
@@ -1914,7 +1939,7 @@ TracePlan trace_plan(const SceneView& V, int32_t n_rays, int32_t any_hit, bool c
     t.lds = trace_lds_bytes(t.lds_entries, any_hit != 0 && !count);
     const bool full = depth <= t.lds_entries;
     t.kfn = batch_kernel(any_hit != 0, count, full, V.has_alpha != 0);
-    t.grid = std::min(trace_grid(reinterpret_cast<const void*>(t.kfn), t.lds), grid_for(std::max(n_rays, 1), kTraceBlock));
+    t.grid = std::min(trace_grid(reinterpret_cast<const void*>(t.kfn), t.lds), trace_blocks(std::max(n_rays, 1), kTraceBlock));
     t.overflow_per_lane = size_t(std::max(0, depth - t.lds_entries));
     return t;
 }
@@ -2246,9 +2271,9 @@ int render_impl(BbScene* scene, const BbCameraDesc* camera, const BbRenderParams
     void (*const k_shade_fn)(SceneView, RenderConsts, PathBufs, int, CacheBufs) = shade_kernel(V, cache != nullptr);
     const ShadowKernel k_shadow = shadow_kernel(count, sk, V.has_alpha != 0, tblock);
     const int g_trace =
-        std::min(trace_grid(reinterpret_cast<const void*>(k_closest), lds, tblock), grid_for(cap, tblock));
+        std::min(trace_grid(reinterpret_cast<const void*>(k_closest), lds, tblock), trace_blocks(cap, tblock));
     const int g_shadow =
-        std::min(trace_grid(reinterpret_cast<const void*>(k_shadow), lds_shadow, tblock), grid_for(cap, tblock));
+        std::min(trace_grid(reinterpret_cast<const void*>(k_shadow), lds_shadow, tblock), trace_blocks(cap, tblock));
     // the overflow area serves both grids (int2-sized entries hold the 4-byte ones too)
     const size_t overflow = sk == kStackSplit ? size_t(depth - lds_entries) : 0;
     // Shadow rays of depth d and closest hits of depth d + 1 read only what
