@@ -171,18 +171,24 @@ struct SceneView
     int32_t has_null_material;
     float root_box[6];  // root node box: min.xyz, max.xyz
     int32_t root_ref;   // the root as a reference (inner record 0, or a leaf)
-    // Two-level records (8 float4 each) for the traversal kernels that keep
+    // Two-level records (64 bytes each) for the traversal kernels that keep
     // no node counters: record of internal node N holds the entries of N's
     // children, an inner child replaced by its own two children (so up to 4
-    // entries: node N's grandchildren, or a child that is a leaf):
-    //   {b0.min.xyz, b0.max.x} {b0.max.yz, b1.min.xy} {b1.min.z, b1.max.xyz}
-    //   {b2.min.xyz, b2.max.x} {b2.max.yz, b3.min.xy} {b3.min.z, b3.max.xyz}
-    //   {ref0, ref1, ref2, ref3} {meta, 0, 0, 0}
+    // entries: node N's grandchildren, or a child that is a leaf).  Their
+    // boxes are rounded outwards to 8 bits per plane on a grid of the record,
+    // planes at p + q 2^e on each axis, packed one byte per entry:
+    //   {p.x, p.y, p.z, e.x | e.y << 8 | e.z << 16 (signed bytes)}
+    //   {min.x, min.y, min.z, order}  {max.x, max.y, max.z, 0}
+    //   {ref0, ref1, ref2, ref3}
     // entries 0, 1 come from child1 (N + 1), entries 2, 3 from child2; an
-    // entry is a two-level record (>= 0) or a leaf (~first slot).  meta:
-    // bits 0-1 N's split axis, 2-3 child1's, 4-5 child2's, bit 6: entry 1
-    // exists (child1 is inner), bit 7: entry 3 exists (child2 is inner).
-    const float4* quads;
+    // entry is a two-level record (>= 0) or a leaf (~first slot), or missing
+    // (INT32_MIN: a child that is a leaf has no second entry).  order: 3 bits
+    // for each octant o of the ray's direction signs (bit a of o: negative
+    // along axis a), at 3 o: child2 comes first (N's split axis), entry 1
+    // comes before entry 0 (child1's), entry 3 before entry 2 (child2's).
+    const uint4* quads;
+    const float4* leaf_box; // 2 per slot, at a leaf's first slot: its exact box {min, 0} {max, 0}
+    float world_abs[3];     // largest finite coordinate of any box, per axis
     int32_t quad_root;        // the root as a two-level reference (record 0, or a leaf)
     int32_t quad_stack_depth; // most stack entries a two-level traversal holds (+ 1)
 };

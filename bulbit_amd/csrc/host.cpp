@@ -6,6 +6,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <cfloat>
 #include <chrono>
 #include <cstdarg>
 #include <cstdio>
@@ -530,6 +531,86 @@ bool textures_to_gpu(const BbSceneDesc& d, std::vector<GpuTexture>& out, std::ve
     return true;
 }
 
+// fn(i) for i in [0, n), on several threads from 2^15 items up; fn(i) writes
+// what belongs to i alone
+template <typename F>
+void for_each_index(int64_t n, F fn)
+{
+    const int64_t threads = std::min<int64_t>({ n >> 15, 8, int64_t(std::max(1u, std::thread::hardware_concurrency())) });
+    auto part = [&](int64_t k, int64_t of) {
+        for (int64_t i = n * k / of; i < n * (k + 1) / of; ++i) fn(i);
+    };
+    std::vector<std::future<void>> rest;
+    for (int64_t k = 1; k < threads; ++k) {
+        try {
+            rest.push_back(std::async(std::launch::async, part, k, threads));
+        } catch (const std::system_error&) { // no thread to be had
+            part(k, threads);
+        }
+    }
+    part(0, std::max<int64_t>(1, threads));
+    for (auto& f : rest) f.get();
+}
+
+uint32_t f2u(float f)
+{
+    uint32_t u;
+    memcpy(&u, &f, 4);
+    return u;
+}
+
+// One axis of a two-level record (SceneView::quads): the grid p + q 2^e and
+// the entries' planes rounded outwards to it, a byte per entry (a missing
+// entry gets an empty range)
+struct QuadGrid
+{
+    float p;
+    int8_t e;
+    uint32_t lo, hi;
+};
+
+QuadGrid quad_grid(const BbBvhNode* const box[4], int axis)
+{
+    QuadGrid g{ 0.0f, 0, 0, 0 };
+    double lo = HUGE_VAL, hi = -HUGE_VAL;
+    bool finite = true;
+    for (int k = 0; k < 4; ++k) {
+        if (!box[k]) continue;
+        finite = finite && std::isfinite(box[k]->bmin[axis]) && std::isfinite(box[k]->bmax[axis]);
+        lo = std::min(lo, double(box[k]->bmin[axis]));
+        hi = std::max(hi, double(box[k]->bmax[axis]));
+    }
+    if (!finite) { // planes beyond every ray: the axis never fails a box
+        g.p = -FLT_MAX;
+        g.e = 127;
+        for (int k = 0; k < 4; ++k)
+            if (box[k]) g.hi |= 255u << (8 * k);
+        return g;
+    }
+    g.p = float(lo); // one of the boxes' planes
+    // 2^e > (hi - lo) / 255, from the exponent bits
+    const double step = (hi - lo) / 255.0;
+    uint64_t bits;
+    memcpy(&bits, &step, 8);
+    const int e = step > 0.0 ? std::max(-126, std::min(127, int(bits >> 52) - 1022)) : 0;
+    bits = uint64_t(1023 - e) << 52; // 2^-e
+    double inv;
+    memcpy(&inv, &bits, 8);
+    for (int k = 0; k < 4; ++k) {
+        uint32_t a = 255, b = 0;
+        if (box[k]) {
+            const double x = (double(box[k]->bmin[axis]) - lo) * inv, y = (double(box[k]->bmax[axis]) - lo) * inv;
+            a = std::min(255u, uint32_t(x));
+            b = uint32_t(y);
+            b = std::min(255u, b + (double(b) < y ? 1u : 0u));
+        }
+        g.lo |= a << (8 * k);
+        g.hi |= b << (8 * k);
+    }
+    g.e = int8_t(e);
+    return g;
+}
+
 } // namespace
 
 bool create_scene(const BbSceneDesc& d, BbScene* s, std::string& err)
@@ -662,9 +743,9 @@ bool create_scene(const BbSceneDesc& d, BbScene* s, std::string& err)
     std::vector<float4> tris(size_t(3) * ns);
     std::vector<int4> slot_shade(ns);
     std::vector<int32_t> slot_light(ns);
-    std::vector<BbBvhNode> nodes = bvh.nodes;
-    bool has_null = false;
-    for (int32_t j = 0; j < ns; ++j) {
+    const std::vector<BbBvhNode>& nodes = bvh.nodes;
+    std::atomic<bool> has_null{ false }, alpha_sphere{ false };
+    for_each_index(ns, [&](int64_t j) {
         int32_t prim = bvh.ordered[j];
         const BbPrimitive& p = d.primitives[prim];
         int32_t prim_bits = prim;
@@ -682,10 +763,7 @@ bool create_scene(const BbSceneDesc& d, BbScene* s, std::string& err)
             tris[3 * size_t(j) + 2] = make_float4(e2.x, e2.y, e2.z, i2f(KIND_TRIANGLE | (alpha ? kSlotAlpha : 0)));
             slot_shade[j] = make_int4(v[0], v[1], v[2], p.material);
         } else {
-            if (p.material >= 0 && mats[p.material].tex_alpha >= 0) {
-                err = "alpha textures on spheres are not supported";
-                return false;
-            }
+            if (p.material >= 0 && mats[p.material].tex_alpha >= 0) alpha_sphere = true;
             int32_t kind = KIND_SPHERE, sidx = p.shape_index;
             float kind_f, sidx_f;
             memcpy(&kind_f, &kind, 4);
@@ -695,6 +773,10 @@ bool create_scene(const BbSceneDesc& d, BbScene* s, std::string& err)
             tris[3 * size_t(j) + 2] = make_float4(0.0f, 0.0f, 0.0f, kind_f);
             slot_shade[j] = make_int4(0, 0, 0, p.material);
         }
+    });
+    if (alpha_sphere) {
+        err = "alpha textures on spheres are not supported";
+        return false;
     }
     // flag the last slot of every leaf, and build the 64-byte inner records:
     // record of internal node i = boxes and references of children i + 1 and
@@ -709,8 +791,8 @@ bool create_scene(const BbSceneDesc& d, BbScene* s, std::string& err)
         }
     auto ref_of = [&](size_t c) { return nodes[c].count == 0 ? inner_index[c] : ~nodes[c].offset; };
     std::vector<float4> inner(size_t(4) * std::max(1, n_inner));
-    for (size_t i = 0; i < nodes.size(); ++i) {
-        if (nodes[i].count != 0) continue;
+    for_each_index(int64_t(nodes.size()), [&](int64_t i) {
+        if (nodes[i].count != 0) return;
         const BbBvhNode& c1 = nodes[i + 1];
         const BbBvhNode& c2 = nodes[size_t(nodes[i].offset)];
         float4* r = &inner[size_t(4) * inner_index[i]];
@@ -718,7 +800,7 @@ bool create_scene(const BbSceneDesc& d, BbScene* s, std::string& err)
         r[1] = make_float4(c1.bmax[1], c1.bmax[2], c2.bmin[0], c2.bmin[1]);
         r[2] = make_float4(c2.bmin[2], c2.bmax[0], c2.bmax[1], c2.bmax[2]);
         r[3] = make_float4(i2f(ref_of(i + 1)), i2f(ref_of(size_t(nodes[i].offset))), i2f(int32_t(nodes[i].axis)), 0.0f);
-    }
+    });
     // two-level records: one for the root and one for every inner node that
     // is an entry of another record (an inner grandchild), numbered in
     // depth-first order; quad_levels = the most records on a root-to-leaf walk
@@ -751,58 +833,76 @@ bool create_scene(const BbSceneDesc& d, BbScene* s, std::string& err)
     }
     const int32_t n_quad = int32_t(quad_order.size());
     auto qref_of = [&](size_t c) { return nodes[c].count == 0 ? quad_index[c] : ~nodes[c].offset; };
-    std::vector<float4> quads(size_t(8) * std::max(1, n_quad), make_float4(0.0f, 0.0f, 0.0f, 0.0f));
-    for (int32_t qi = 0; qi < n_quad; ++qi) {
+    // the records, then every leaf's exact box (one upload)
+    const size_t quad_vecs = size_t(4) * std::max(1, n_quad);
+    std::vector<uint4> quads(quad_vecs + size_t(2) * ns, make_uint4(0, 0, 0, 0));
+    std::atomic<bool> bad_axis{ false };
+    for_each_index(n_quad, [&](int64_t qi) {
         const size_t nn = size_t(quad_order[qi]);
         const size_t kids[2] = { nn + 1, size_t(nodes[nn].offset) };
         size_t ent[4] = { 0, 0, 0, 0 };
         bool has[4] = { true, false, true, false };
-        int32_t meta = int32_t(nodes[nn].axis);
+        int32_t axes[3] = { int32_t(nodes[nn].axis), 0, 0 }; // N's, child1's, child2's
+        bool inner_child[2] = { false, false };
         for (int c = 0; c < 2; ++c) {
             const size_t k = kids[c];
             if (nodes[k].count == 0) {
                 ent[2 * c] = k + 1;
                 ent[2 * c + 1] = size_t(nodes[k].offset);
                 has[2 * c + 1] = true;
-                meta |= int32_t(nodes[k].axis) << (2 + 2 * c);
-                meta |= 1 << (6 + c);
+                inner_child[c] = true;
+                axes[1 + c] = int32_t(nodes[k].axis);
             } else {
                 ent[2 * c] = k;
             }
         }
-        float box[4][6] = {};
-        int32_t ref[4] = { 0, 0, 0, 0 };
+        if (axes[0] > 2 || axes[1] > 2 || axes[2] > 2) {
+            bad_axis = true;
+            return;
+        }
+        const BbBvhNode* box[4];
+        int32_t ref[4];
         for (int e = 0; e < 4; ++e) {
-            if (!has[e]) continue;
-            const BbBvhNode& b = nodes[ent[e]];
-            for (int a = 0; a < 3; ++a) {
-                box[e][a] = b.bmin[a];
-                box[e][3 + a] = b.bmax[a];
-            }
-            ref[e] = qref_of(ent[e]);
+            box[e] = has[e] ? &nodes[ent[e]] : nullptr;
+            ref[e] = has[e] ? qref_of(ent[e]) : INT32_MIN;
         }
-        float4* r = &quads[size_t(8) * qi];
-        for (int h = 0; h < 2; ++h) {
-            const float* b0 = box[2 * h];
-            const float* b1 = box[2 * h + 1];
-            r[3 * h + 0] = make_float4(b0[0], b0[1], b0[2], b0[3]);
-            r[3 * h + 1] = make_float4(b0[4], b0[5], b1[0], b1[1]);
-            r[3 * h + 2] = make_float4(b1[2], b1[3], b1[4], b1[5]);
-        }
-        r[6] = make_float4(i2f(ref[0]), i2f(ref[1]), i2f(ref[2]), i2f(ref[3]));
-        r[7] = make_float4(i2f(meta), 0.0f, 0.0f, 0.0f);
+        QuadGrid g[3];
+        for (int a = 0; a < 3; ++a) g[a] = quad_grid(box, a);
+        // bit 3 o for every octant o that is negative along the axis
+        constexpr uint32_t kNegative[3] = { 0x208208u, 0x240240u, 0x249000u };
+        const uint32_t order = kNegative[axes[0]] | (inner_child[0] ? kNegative[axes[1]] << 1 : 0u) |
+                               (inner_child[1] ? kNegative[axes[2]] << 2 : 0u);
+        uint4* r = &quads[size_t(4) * qi];
+        r[0] = make_uint4(f2u(g[0].p), f2u(g[1].p), f2u(g[2].p),
+                          uint32_t(uint8_t(g[0].e)) | uint32_t(uint8_t(g[1].e)) << 8 | uint32_t(uint8_t(g[2].e)) << 16);
+        r[1] = make_uint4(g[0].lo, g[1].lo, g[2].lo, order);
+        r[2] = make_uint4(g[0].hi, g[1].hi, g[2].hi, 0);
+        r[3] = make_uint4(uint32_t(ref[0]), uint32_t(ref[1]), uint32_t(ref[2]), uint32_t(ref[3]));
+    });
+    if (bad_axis) {
+        err = "internal error: BVH split axis out of range";
+        return false;
+    }
+    // the leaves' boxes, and the largest coordinates
+    float world_abs[3] = { 0.0f, 0.0f, 0.0f };
+    for (const BbBvhNode& nd : nodes) {
+        if (nd.count == 0) continue;
+        uint4* box = &quads[quad_vecs + 2 * size_t(nd.offset)];
+        box[0] = make_uint4(f2u(nd.bmin[0]), f2u(nd.bmin[1]), f2u(nd.bmin[2]), 0);
+        box[1] = make_uint4(f2u(nd.bmax[0]), f2u(nd.bmax[1]), f2u(nd.bmax[2]), 0);
+        for (int a = 0; a < 3; ++a)
+            for (const float c : { nd.bmin[a], nd.bmax[a] })
+                if (std::isfinite(c)) world_abs[a] = std::max(world_abs[a], std::fabs(c));
     }
 
     // every reference the kernels follow stays inside its array
     auto ref_ok = [&](int32_t ref) { return ref >= 0 ? ref < n_inner : (~ref >= 0 && ~ref < ns); };
     auto qref_ok = [&](int32_t ref) { return ref >= 0 ? ref < n_quad : (~ref >= 0 && ~ref < ns); };
     for (int32_t k = 0; k < n_quad; ++k) {
-        const float4 rr = quads[size_t(8) * k + 6];
-        const int32_t meta = f2i(quads[size_t(8) * k + 7].x);
-        const int32_t rs[4] = { f2i(rr.x), f2i(rr.y), f2i(rr.z), f2i(rr.w) };
-        const bool has1 = (meta >> 6) & 1, has3 = (meta >> 7) & 1;
-        if (!qref_ok(rs[0]) || !qref_ok(rs[2]) || (has1 && !qref_ok(rs[1])) || (has3 && !qref_ok(rs[3])) ||
-            (meta & 3) == 3 || ((meta >> 2) & 3) == 3 || ((meta >> 4) & 3) == 3) {
+        const uint4 rr = quads[size_t(4) * k + 3];
+        const int32_t rs[4] = { int32_t(rr.x), int32_t(rr.y), int32_t(rr.z), int32_t(rr.w) };
+        auto second_ok = [&](int32_t ref) { return ref == INT32_MIN || qref_ok(ref); }; // may be missing
+        if (!qref_ok(rs[0]) || !qref_ok(rs[2]) || !second_ok(rs[1]) || !second_ok(rs[3])) {
             err = "internal error: two-level BVH record out of range";
             return false;
         }
@@ -821,10 +921,10 @@ bool create_scene(const BbSceneDesc& d, BbScene* s, std::string& err)
     }
 
     std::vector<float4> normals(std::max(1, d.n_vertices)), tangents(std::max(1, d.n_vertices));
-    for (int32_t i = 0; i < d.n_vertices; ++i) {
+    for_each_index(d.n_vertices, [&](int64_t i) {
         normals[i] = make_float4(d.normals[3 * i], d.normals[3 * i + 1], d.normals[3 * i + 2], 0.0f);
         tangents[i] = make_float4(d.tangents[3 * i], d.tangents[3 * i + 1], d.tangents[3 * i + 2], 0.0f);
-    }
+    });
 
     SceneView& V = s->view;
     hipGetDevice(&s->device);
@@ -836,8 +936,11 @@ bool create_scene(const BbSceneDesc& d, BbScene* s, std::string& err)
     V.root_ref = ref_of(0);
     if (!upload(s, quads.data(), quads.size(), &V.quads, err)) return false;
     V.quad_root = qref_of(0);
-    // each record pushes at most 3 entries
+    // each record leaves at most 3 entries on the stack beside the one taken
+    // next, which is pushed too
     V.quad_stack_depth = 3 * quad_levels + 1;
+    V.leaf_box = reinterpret_cast<const float4*>(V.quads + quad_vecs);
+    for (int a = 0; a < 3; ++a) V.world_abs[a] = world_abs[a];
     if (!upload(s, tris.data(), tris.size(), &V.tris, err)) return false;
     if (!upload(s, slot_shade.data(), slot_shade.size(), &V.slot_shade, err)) return false;
     if (!upload(s, slot_light.data(), slot_light.size(), &V.slot_light, err)) return false;

@@ -51,6 +51,19 @@ constexpr int kShadeBlock = 256;
 #endif
 constexpr int kReservoir = BB_RESERVOIR; // queries a traversal wave claims per atomic
 constexpr int kFirstChunkMin = 8; // fewest queries a wave starts with
+// a wave tests leaves once kLeafMin lanes wait at one, or once the lanes at
+// inner nodes are at most kLeafShare times as many (1080p frame of 64 spp,
+// min / share: 1 / 64, the leaves at once, 77.7 ms; 8 / 4 76.1, 16 / 4 75.9,
+// 16 / 2 75.7, 24 / 1 75.8, 32 / 1 75.7; the 1-spp preview 2.24 ms at once,
+// 2.22 with 16 / 2, 2.25 with 32 / 1)
+constexpr int kLeafMin = 16;
+constexpr int kLeafShare = 2;
+// waves per SIMD the traversal kernels are built for (72 VGPRs): left to
+// itself the compiler took 87 and five waves fitted (72.6 ms per 1080p frame
+// of 64 spp; six 70.1, seven 68.8, eight, with spills, 70.8).  Not the
+// kernels with the alpha test, which spill (textured 801 x 451 frame of 8
+// spp: 6.6 ms without the bound, 7.1 at six, 7.6 at seven).
+constexpr int kTraceWaves = 7;
 constexpr int kLdsCdfEntries = 2049; // lights whose CDF the shading kernel keeps in LDS (up to 2048)
 constexpr int kMaxGridBlocks = 256 * 32;
 
@@ -163,6 +176,11 @@ struct Lane
     f3 o, d, inv, dn;
     float l, t_min, t_max;
     bool n0, n1, n2;
+    // two-level records (quad_ray): the inverse direction and offsets of
+    // their slab distances, and the bit position of the ray's octant in a
+    // record's order word
+    f3 qinv, qnear, qfar;
+    uint32_t oct;
     int32_t sp, cur;
     int32_t hit_slot;
     float hit_t, hit_u, hit_v;
@@ -220,10 +238,6 @@ BB_D void lane_start(Lane& L, f3 o, f3 d, float t_min, float t_max)
     L.d = d;
     L.t_min = t_min;
     L.t_max = t_max;
-    L.inv = mk3(1.0f / d.x, 1.0f / d.y, 1.0f / d.z);
-    L.n0 = L.inv.x < 0.0f;
-    L.n1 = L.inv.y < 0.0f;
-    L.n2 = L.inv.z < 0.0f;
     L.dn = d;
     L.l = normalize_m(L.dn);
     L.sp = 0;
@@ -232,37 +246,125 @@ BB_D void lane_start(Lane& L, f3 o, f3 d, float t_min, float t_max)
     L.hit_t = L.hit_u = L.hit_v = 0.0f;
 }
 
+// The ray's constants for the boxes of two-level records, whose slab
+// distances are
+//   near = fma(q, s inv, fma(p, inv, qnear)),  far likewise with qfar
+// for a plane at p + q s: -o inv with a margin M taken off (near) or added
+// (far), so that each box test passes whenever the exact one (box_part) of a
+// box inside does.  In units of u = 2^-24 (|o| + w) |inv|, w the largest
+// coordinate of the scene on the axis, the errors are: the reciprocal two,
+// -o inv - M one, the inner fma one, the outer one, box_part's reciprocal
+// one, subtraction and product two; the quantized planes lie outside the
+// box's.  M is over 13 u.
+// An axis the direction hardly moves along has an inverse so large that
+// o inv would overflow or cancel; there |inv| is cut to 2^40 times the
+// smallest of the three and M taken from the largest of the three scene
+// extents.  M alone is then some 2^19 times the distance at which the ray
+// leaves the scene, so a slab around the origin never fails, a slab the
+// origin lies outside of by more than M's share still does, and no box is
+// decided on that axis in margin_pass's certain form.  NaN slab distances
+// (NaN rays) are ignored, as box_part ignores them.  Returns the largest
+// coordinate the ray starts from or may meet.
+BB_D float quad_ray(const SceneView& S, Lane& L)
+{
+    const f3 inv = mk3(__builtin_amdgcn_rcpf(L.d.x), __builtin_amdgcn_rcpf(L.d.y), __builtin_amdgcn_rcpf(L.d.z));
+    L.n0 = inv.x < 0.0f;
+    L.n1 = inv.y < 0.0f;
+    L.n2 = inv.z < 0.0f;
+    L.oct = (L.n0 ? 3u : 0u) + (L.n1 ? 6u : 0u) + (L.n2 ? 12u : 0u);
+    const float ax = fabsf(inv.x), ay = fabsf(inv.y), az = fabsf(inv.z);
+    const float sx = fabsf(L.o.x) + S.world_abs[0], sy = fabsf(L.o.y) + S.world_abs[1],
+                sz = fabsf(L.o.z) + S.world_abs[2];
+    const float smax = fmaxf(fmaxf(sx, sy), sz);
+    const float most = fminf(fminf(fminf(ax, ay), az) * 0x1p40f, 1e36f * __builtin_amdgcn_rcpf(smax));
+    const bool cx = ax > most, cy = ay > most, cz = az > most;
+    const float bx = cx ? most : ax, by = cy ? most : ay, bz = cz ? most : az;
+    L.qinv = mk3(copysignf(bx, inv.x), copysignf(by, inv.y), copysignf(bz, inv.z));
+    const float mx = fmaf((cx ? smax : sx) * bx, 8e-7f, 1e-36f), my = fmaf((cy ? smax : sy) * by, 8e-7f, 1e-36f),
+                mz = fmaf((cz ? smax : sz) * bz, 8e-7f, 1e-36f);
+    L.qnear = mk3(fmaf(-L.o.x, L.qinv.x, -mx), fmaf(-L.o.y, L.qinv.y, -my), fmaf(-L.o.z, L.qinv.z, -mz));
+    L.qfar = mk3(fmaf(-L.o.x, L.qinv.x, mx), fmaf(-L.o.y, L.qinv.y, my), fmaf(-L.o.z, L.qinv.z, mz));
+    return smax;
+}
+
+// A box test with the ray's margins: `certain` false, it passes whenever the
+// exact test of the box, or of one inside it, does; true, it passes only
+// when the exact test of the box does
+BB_D bool margin_pass(const Lane& L, f3 bmin, f3 bmax, float t_max, bool certain)
+{
+    const f3 kn = certain ? L.qfar : L.qnear, kf = certain ? L.qnear : L.qfar;
+    const float lo = fmaxf(fmaxf(fmaf(L.n0 ? bmax.x : bmin.x, L.qinv.x, kn.x), fmaf(L.n1 ? bmax.y : bmin.y, L.qinv.y, kn.y)),
+                           fmaf(L.n2 ? bmax.z : bmin.z, L.qinv.z, kn.z));
+    const float hi = fminf(fminf(fmaf(L.n0 ? bmin.x : bmax.x, L.qinv.x, kf.x), fmaf(L.n1 ? bmin.y : bmax.y, L.qinv.y, kf.y)),
+                           fmaf(L.n2 ? bmin.z : bmax.z, L.qinv.z, kf.z));
+    // written so that a NaN (no axis left) is a pass only when uncertain ones are
+    return certain ? (L.t_min <= hi) & (lo <= hi) & (lo <= t_max) : !((L.t_min > hi) | (lo > hi) | (lo > t_max));
+}
+
+// RayCast's test of a box
+BB_D bool exact_pass(const Lane& L, f3 bmin, f3 bmax, float t_max)
+{
+    const f3 inv = mk3(1.0f / L.d.x, 1.0f / L.d.y, 1.0f / L.d.z);
+    return box_pass(box_part(bmin, bmax, L.o, L.t_min, inv, inv.x < 0.0f, inv.y < 0.0f, inv.z < 0.0f), t_max);
+}
+
+// Whether RayCast visits the leaf whose first slot is `slot` with this t_max:
+// its exact box test, skipped when the margins already decide it
+BB_D bool leaf_visited(const SceneView& S, const Lane& L, int32_t slot, float t_max)
+{
+    const float4 a = S.leaf_box[2 * size_t(slot)], b = S.leaf_box[2 * size_t(slot) + 1];
+    const f3 bmin = mk3(a.x, a.y, a.z), bmax = mk3(b.x, b.y, b.z);
+    return margin_pass(L, bmin, bmax, t_max, true) || exact_pass(L, bmin, bmax, t_max);
+}
+
 // the root is the first node RayCast takes off its stack and box-tests
 template <bool COUNT>
 BB_D void lane_root(const SceneView& S, Lane& L, TraceCount& c)
 {
-    if (COUNT) c.nodes++;
-    const BoxHit h = box_part(mk3(S.root_box[0], S.root_box[1], S.root_box[2]),
-                              mk3(S.root_box[3], S.root_box[4], S.root_box[5]), L.o, L.t_min, L.inv, L.n0, L.n1,
-                              L.n2);
-    L.cur = box_pass(h, L.t_max) ? (COUNT ? S.root_ref : S.quad_root) : kNoRef;
+    const f3 bmin = mk3(S.root_box[0], S.root_box[1], S.root_box[2]);
+    const f3 bmax = mk3(S.root_box[3], S.root_box[4], S.root_box[5]);
+    if constexpr (COUNT) {
+        c.nodes++;
+        L.inv = mk3(1.0f / L.d.x, 1.0f / L.d.y, 1.0f / L.d.z);
+        L.n0 = L.inv.x < 0.0f;
+        L.n1 = L.inv.y < 0.0f;
+        L.n2 = L.inv.z < 0.0f;
+        const BoxHit h = box_part(bmin, bmax, L.o, L.t_min, L.inv, L.n0, L.n1, L.n2);
+        L.cur = box_pass(h, L.t_max) ? S.root_ref : kNoRef;
+    } else {
+        const float smax = quad_ray(S, L);
+        bool pass = margin_pass(L, bmin, bmax, L.t_max, false);
+        if (!(smax < 1e30f)) pass = exact_pass(L, bmin, bmax, L.t_max); // no margin holds: an infinite ray ends here
+        L.cur = pass ? S.quad_root : kNoRef;
+    }
 }
 
 // Traversal stack: entries [0, lds_entries) in LDS ([entry][thread] layout,
 // conflict-free for a wave), deeper entries in a global overflow area
 // ([entry][global thread]); cap = BVH depth + 2 bounds every push.  An entry
-// is a (node reference, entry distance) pair (int2), or the reference alone
+// is a (node reference, entry distance) pair (i2v), or the reference alone
 // (int) for any-hit queries without counters, whose t_max never changes
-// while they run, so the pop-time `lo > t_max` check cannot fail.
+// while they run, so the pop-time `lo > t_max` check cannot fail.  The three
+// places keep their own address spaces: through one generic pointer every
+// push and pop was a flat access, behind 64-bit address arithmetic and a
+// wait on both memory counters.
+typedef int i2v __attribute__((ext_vector_type(2)));
+#define BB_LDS __attribute__((address_space(3)))
+
 template <typename E>
 struct TraceStack
 {
-    E* lds;
+    BB_LDS E* lds; // the lane's first entry; entries are a block's threads apart
     E* gbl;
+    E* priv;
     int32_t lds_entries;
-    int32_t lstride; // LDS entries of one lane are this far apart (the block size)
     int32_t gstride;
     int32_t cap;
 };
 
 // stack entries of a query kind
 template <bool ANY, bool COUNT>
-using StackEntry = typename std::conditional<ANY && !COUNT, int, int2>::type;
+using StackEntry = typename std::conditional<ANY && !COUNT, int, i2v>::type;
 
 // Where a lane's traversal stack lives (the SK template parameter):
 //   kStackSplit    the first lds_entries entries in LDS, deeper ones in the
@@ -278,22 +380,32 @@ enum : int
 };
 constexpr int kScratchStackEntries = 64; // cap of the private-array stack
 
-template <int SK, typename E>
+template <int SK, int BLOCK, typename E>
 BB_D void stack_put(const TraceStack<E>& s, int32_t sp, E v)
 {
-    if (SK == kStackScratch)
-        s.lds[sp] = v;
-    else if (SK == kStackLds || sp < s.lds_entries)
-        s.lds[sp * s.lstride] = v;
-    else
-        s.gbl[(sp - s.lds_entries) * s.gstride] = v;
+    if constexpr (SK == kStackScratch) {
+        s.priv[sp] = v;
+    } else if constexpr (SK == kStackLds) {
+        s.lds[sp * BLOCK] = v;
+    } else {
+        if (sp < s.lds_entries)
+            s.lds[sp * BLOCK] = v;
+        else
+            s.gbl[size_t(sp - s.lds_entries) * s.gstride] = v;
+    }
 }
 
-template <int SK, typename E>
+template <int SK, int BLOCK, typename E>
 BB_D E stack_get(const TraceStack<E>& s, int32_t sp)
 {
-    if (SK == kStackScratch) return s.lds[sp];
-    return (SK == kStackLds || sp < s.lds_entries) ? s.lds[sp * s.lstride] : s.gbl[(sp - s.lds_entries) * s.gstride];
+    if constexpr (SK == kStackScratch) return s.priv[sp];
+    if constexpr (SK == kStackLds) return s.lds[sp * BLOCK];
+    E v;
+    if (sp < s.lds_entries)
+        v = s.lds[sp * BLOCK];
+    else
+        v = s.gbl[size_t(sp - s.lds_entries) * s.gstride];
+    return v;
 }
 
 // a far child whose t_max-independent test failed, kept on the stack only
@@ -301,35 +413,50 @@ BB_D E stack_get(const TraceStack<E>& s, int32_t sp)
 // (a signalling-NaN bit pattern: no arithmetic result has it)
 constexpr int32_t kFailedLo = 0x7fbfffff;
 
-// One step of RayCast for one lane.
-//
-// Expanding an inner record tests both children's boxes from the parent's
-// 64 bytes.  RayCast pushes the far child, then tests the near child with
-// the current t_max: the near test here is that same test.  The far child is
-// tested by RayCast when popped, with the t_max of that moment; here its
-// t_max-independent part and entry distance are computed now, a child that
-// fails already is not pushed (it would fail then too), and the pop applies
-// the remaining `lo > t_max` check with the then-current t_max.  So the same
-// nodes are expanded in the same order with the same outcomes, and leaves
-// test their primitives in stored order (the callbacks of BVH::Intersect /
-// IntersectAny, src/accel/bvh.cpp:299-361).  With COUNT, every far child is
-// pushed and counted when popped, which reproduces RayCast's node-test count.
-// Returns true when the lane's query is finished.
-// An entry of a two-level record: its reference and box test
+// Expands an inner record (one level) for one lane, for the kernels that
+// count RayCast's node tests.  RayCast pushes the far child, then tests the
+// near child with the current t_max: the near test here is that same test.
+// The far child is tested by RayCast when popped, with the t_max of that
+// moment; here its t_max-independent part and entry distance are computed
+// now and it is pushed either way, so that it is counted when popped.  The
+// near child, or kNoRef, becomes the lane's next node.
+template <bool ANY, int SK, int BLOCK>
+BB_D void inner_expand(const SceneView& S, Lane& L, const TraceStack<i2v>& stk, TraceCount& c, int* err)
+{
+    const float4* r = S.inner + 4 * size_t(L.cur);
+    const float4 a = r[0], b = r[1], e = r[2], m = r[3];
+    const BoxHit h1 = box_part(mk3(a.x, a.y, a.z), mk3(a.w, b.x, b.y), L.o, L.t_min, L.inv, L.n0, L.n1, L.n2);
+    const BoxHit h2 = box_part(mk3(b.z, b.w, e.x), mk3(e.y, e.z, e.w), L.o, L.t_min, L.inv, L.n0, L.n1, L.n2);
+    const int32_t axis = __float_as_int(m.z);
+    const bool neg = axis == 0 ? L.n0 : (axis == 1 ? L.n1 : L.n2);
+    const int32_t near_ref = __float_as_int(neg ? m.y : m.x);
+    const int32_t far_ref = __float_as_int(neg ? m.x : m.y);
+    const BoxHit hn = neg ? h2 : h1;
+    const BoxHit hf = neg ? h1 : h2;
+    if (L.sp >= stk.cap) {
+        atomicOr(err, 1);
+        L.sp = 0;
+        L.cur = kNoRef;
+        return;
+    }
+    stack_put<SK, BLOCK>(stk, L.sp, i2v{ far_ref, hf.ok ? __float_as_int(hf.lo) : kFailedLo });
+    ++L.sp;
+    c.nodes++;
+    L.cur = box_pass(hn, L.t_max) ? near_ref : kNoRef;
+}
+
+// An entry of a two-level record whose box test passed (ref), or kNoRef
 struct QEnt
 {
     int32_t ref;
-    BoxHit h;
+    float lo; // the box's entry distance
 };
 
-BB_D QEnt qsel(bool c, QEnt a, QEnt b)
-{
-    QEnt r;
-    r.ref = c ? a.ref : b.ref;
-    r.h.ok = c ? a.h.ok : b.h.ok;
-    r.h.lo = c ? a.h.lo : b.h.lo;
-    return r;
-}
+BB_D QEnt qsel(bool c, QEnt a, QEnt b) { return QEnt{ c ? a.ref : b.ref, c ? a.lo : b.lo }; }
+
+// byte `E` of a packed row as a float
+template <int E>
+BB_D float qbyte(uint32_t row) { return float((row >> (8 * E)) & 0xffu); }
 
 // Expands a two-level record (SceneView::quads) for one lane.  RayCast at
 // the record's node N tests N's near child now and pushes the far one; at
@@ -337,177 +464,187 @@ BB_D QEnt qsel(bool c, QEnt a, QEnt b)
 // one.  Here the up-to-four entries (grandchildren, or a child that is a
 // leaf) are ordered the same way from the ray's direction signs: near
 // child's near and far entry, then far child's near and far entry.  The
-// first is tested now and the others are pushed in reverse, each with its
-// entry distance for the pop-time `lo > t_max` check.  That visits the same
-// leaves in the same order with the same t_max as RayCast: no leaf lies
-// between a child's test and its near grandchild's, so both meet the same
-// t_max, and a grandchild's box lies inside its parent's, so its slab
-// interval lies inside the parent's (the float slab distances are monotone
-// in the plane coordinates, NaN counting as ignored) and it fails whenever
-// the parent would.  Only the node-test count differs, so the counting
-// kernels keep the one-level records.
-template <bool ANY, int SK>
-BB_D bool quad_expand(const SceneView& S, Lane& L, const TraceStack<StackEntry<ANY, false>>& stk, int* err)
+// first that passes is next and the others that pass are pushed in reverse,
+// each with its entry distance for the pop-time `lo > t_max` check.
+//
+// The boxes are the entries' own boxes rounded outwards to 8 bits per plane,
+// and tested with a margin (quad_ray), so an entry passes whenever RayCast's
+// test of it or of any leaf below it does: every leaf that RayCast visits is
+// visited here, in the same order and, since RayCast's t_max only shrinks,
+// with the same t_max.  A leaf RayCast would not have visited can change
+// nothing unless one of its primitives is accepted, and before a primitive
+// is accepted the leaf's exact box is tested (leaf_visited): a leaf's box
+// lies inside its ancestors', whose slab intervals are then no smaller (the
+// float slab distances are monotone in the plane coordinates, NaN counting
+// as ignored), so that one test decides whether RayCast reaches the leaf.
+// Hits are RayCast's bit for bit; only the node-test count differs, so the
+// counting kernels keep the one-level records.
+//
+// Bound by VALU issue where rays diverge (1.1 instructions per issue slot at
+// the second closest hits of the 1080p frame of 64 spp, 45 of 64 lanes at a
+// node), then by loads.  Tried on that frame (start of the split: 89.0 ms):
+// float planes, four box corners per entry read by address instead of
+// selected by sign, typed stacks and leaves in their own phase 75.6 ms; these
+// 64-byte records, four loads instead of eight, 74.1; no exact divisions at a
+// ray's start, pushes without branches 72.6, 72 VGPRs for seven waves 68.7,
+// all entries pushed and the next one popped, any order for shadow rays 67.6
+// (68.4 without the pixel-major path order).  Half-precision planes that need
+// no conversions (80 bytes, 24 fewer VALU per record) were slower, 72.9.
+template <bool ANY, int SK, int BLOCK>
+BB_D void quad_expand(const SceneView& S, Lane& L, const TraceStack<StackEntry<ANY, false>>& stk, int* err)
 {
     constexpr bool kSlim = std::is_same<StackEntry<ANY, false>, int>::value;
-    const float4* r = S.quads + 8 * L.cur;
-    const float4 q0 = r[0], q1 = r[1], q2 = r[2], q3 = r[3], q4 = r[4], q5 = r[5], q6 = r[6], q7 = r[7];
-    // the record's 128 bytes in one round trip
-    asm volatile("" ::"v"(q0.x), "v"(q0.y), "v"(q0.z), "v"(q0.w), "v"(q1.x), "v"(q1.y), "v"(q1.z), "v"(q1.w),
-                 "v"(q2.x), "v"(q2.y), "v"(q2.z), "v"(q2.w), "v"(q3.x), "v"(q3.y), "v"(q3.z), "v"(q3.w), "v"(q4.x),
-                 "v"(q4.y), "v"(q4.z), "v"(q4.w), "v"(q5.x), "v"(q5.y), "v"(q5.z), "v"(q5.w), "v"(q6.x), "v"(q6.y),
-                 "v"(q6.z), "v"(q6.w), "v"(q7.x));
-    const int32_t meta = __float_as_int(q7.x);
-    const bool has1 = (meta >> 6) & 1, has3 = (meta >> 7) & 1;
-    QEnt e0, e1, e2, e3;
-    e0.ref = __float_as_int(q6.x);
-    e1.ref = __float_as_int(q6.y);
-    e2.ref = __float_as_int(q6.z);
-    e3.ref = __float_as_int(q6.w);
-    e0.h = box_part(mk3(q0.x, q0.y, q0.z), mk3(q0.w, q1.x, q1.y), L.o, L.t_min, L.inv, L.n0, L.n1, L.n2);
-    e1.h = box_part(mk3(q1.z, q1.w, q2.x), mk3(q2.y, q2.z, q2.w), L.o, L.t_min, L.inv, L.n0, L.n1, L.n2);
-    e2.h = box_part(mk3(q3.x, q3.y, q3.z), mk3(q3.w, q4.x, q4.y), L.o, L.t_min, L.inv, L.n0, L.n1, L.n2);
-    e3.h = box_part(mk3(q4.z, q4.w, q5.x), mk3(q5.y, q5.z, q5.w), L.o, L.t_min, L.inv, L.n0, L.n1, L.n2);
-    e1.h.ok = e1.h.ok && has1;
-    e3.h.ok = e3.h.ok && has3;
-    const int32_t aN = meta & 3, aA = (meta >> 2) & 3, aB = (meta >> 4) & 3;
-    const bool nN = aN == 0 ? L.n0 : (aN == 1 ? L.n1 : L.n2);
-    const bool nA = aA == 0 ? L.n0 : (aA == 1 ? L.n1 : L.n2);
-    const bool nB = aB == 0 ? L.n0 : (aB == 1 ? L.n1 : L.n2);
-    // each child's entries in near-far order (child2 is near when d[axis] < 0)
-    const bool sA = has1 && nA, sB = has3 && nB;
-    const QEnt a_near = qsel(sA, e1, e0), a_far = qsel(sA, e0, e1);
-    const QEnt b_near = qsel(sB, e3, e2), b_far = qsel(sB, e2, e3);
-    const QEnt x0 = qsel(nN, b_near, a_near), x1 = qsel(nN, b_far, a_far);
-    const QEnt x2 = qsel(nN, a_near, b_near), x3 = qsel(nN, a_far, b_far);
-    if (L.sp + 3 > stk.cap) {
-        atomicOr(err, 1);
-        return true;
-    }
-    // pushed only when they pass with the current t_max (t_max only shrinks)
-    if (box_pass(x3.h, L.t_max)) {
-        if constexpr (kSlim)
-            stack_put<SK>(stk, L.sp, x3.ref);
-        else
-            stack_put<SK>(stk, L.sp, make_int2(x3.ref, __float_as_int(x3.h.lo)));
-        ++L.sp;
-    }
-    if (box_pass(x2.h, L.t_max)) {
-        if constexpr (kSlim)
-            stack_put<SK>(stk, L.sp, x2.ref);
-        else
-            stack_put<SK>(stk, L.sp, make_int2(x2.ref, __float_as_int(x2.h.lo)));
-        ++L.sp;
-    }
-    if (box_pass(x1.h, L.t_max)) {
-        if constexpr (kSlim)
-            stack_put<SK>(stk, L.sp, x1.ref);
-        else
-            stack_put<SK>(stk, L.sp, make_int2(x1.ref, __float_as_int(x1.h.lo)));
-        ++L.sp;
-    }
-    if (box_pass(x0.h, L.t_max)) {
-        L.cur = x0.ref;
-        return false;
+    const uint4* r = S.quads + 4 * size_t(uint32_t(L.cur));
+    const uint4 w0 = r[0], w1 = r[1], w2 = r[2], rf = r[3];
+    // the record's 64 bytes in one round trip
+    asm volatile("" ::"v"(w0.x), "v"(w1.x), "v"(w2.x), "v"(rf.x));
+    const float px = __uint_as_float(w0.x), py = __uint_as_float(w0.y), pz = __uint_as_float(w0.z);
+    const float sx = __builtin_amdgcn_ldexpf(L.qinv.x, int8_t(w0.w)),
+                sy = __builtin_amdgcn_ldexpf(L.qinv.y, int8_t(w0.w >> 8)),
+                sz = __builtin_amdgcn_ldexpf(L.qinv.z, int8_t(w0.w >> 16));
+    const float anx = fmaf(px, L.qinv.x, L.qnear.x), afx = fmaf(px, L.qinv.x, L.qfar.x);
+    const float any = fmaf(py, L.qinv.y, L.qnear.y), afy = fmaf(py, L.qinv.y, L.qfar.y);
+    const float anz = fmaf(pz, L.qinv.z, L.qnear.z), afz = fmaf(pz, L.qinv.z, L.qfar.z);
+    // the rows of planes the ray meets first and last
+    const uint32_t nx = L.n0 ? w2.x : w1.x, fx = L.n0 ? w1.x : w2.x;
+    const uint32_t ny = L.n1 ? w2.y : w1.y, fy = L.n1 ? w1.y : w2.y;
+    const uint32_t nz = L.n2 ? w2.z : w1.z, fz = L.n2 ? w1.z : w2.z;
+    const uint32_t order = w1.w;
+    auto test = [&](auto e, uint32_t ref) {
+        constexpr int E = decltype(e)::value;
+        const float lo = fmaxf(fmaxf(fmaf(qbyte<E>(nx), sx, anx), fmaf(qbyte<E>(ny), sy, any)),
+                               fmaf(qbyte<E>(nz), sz, anz));
+        const float hi = fminf(fminf(fmaf(qbyte<E>(fx), sx, afx), fmaf(qbyte<E>(fy), sy, afy)),
+                               fmaf(qbyte<E>(fz), sz, afz));
+        const bool fail = (L.t_min > hi) | (lo > hi) | (lo > L.t_max);
+        return QEnt{ fail ? kNoRef : int32_t(ref), lo };
+    };
+    const QEnt e0 = test(std::integral_constant<int, 0>{}, rf.x);
+    const QEnt e1 = test(std::integral_constant<int, 1>{}, rf.y);
+    const QEnt e2 = test(std::integral_constant<int, 2>{}, rf.z);
+    const QEnt e3 = test(std::integral_constant<int, 3>{}, rf.w);
+    QEnt x0 = e0, x1 = e1, x2 = e2, x3 = e3;
+    // (any hit will do for a shadow ray, in any order)
+    if constexpr (!kSlim) {
+        // near-far order for the ray's octant: bit 0 child2 first, bits 1 and 2
+        // the second entry of child1 and of child2 first
+        const uint32_t od = order >> L.oct;
+        const bool nN = od & 1u, sA = od & 2u, sB = od & 4u;
+        const QEnt a_near = qsel(sA, e1, e0), a_far = qsel(sA, e0, e1);
+        const QEnt b_near = qsel(sB, e3, e2), b_far = qsel(sB, e2, e3);
+        x0 = qsel(nN, b_near, a_near);
+        x1 = qsel(nN, b_far, a_far);
+        x2 = qsel(nN, a_near, b_near);
+        x3 = qsel(nN, a_far, b_far);
     }
     L.cur = kNoRef;
-    return false;
-}
-
-template <bool ANY, bool COUNT, int SK, bool ALPHA>
-BB_D bool trace_step(const SceneView& S, Lane& L, const TraceStack<StackEntry<ANY, COUNT>>& stk, TraceCount& c,
-                     int* err)
-{
-    constexpr bool kSlim = std::is_same<StackEntry<ANY, COUNT>, int>::value;
-    if (!COUNT && L.cur >= 0) {
-        // two-level records (no node counters kept)
-        if constexpr (!COUNT) {
-            if (quad_expand<ANY, SK>(S, L, stk, err)) return true;
-            if (L.cur != kNoRef) return false;
-        }
-    } else if (L.cur >= 0) {
-        const float4* r = S.inner + 4 * L.cur;
-        const float4 a = r[0], b = r[1], e = r[2], m = r[3];
-        // the record's 64 bytes in one round trip
-        asm volatile("" ::"v"(a.x), "v"(a.y), "v"(a.z), "v"(a.w), "v"(b.x), "v"(b.y), "v"(b.z), "v"(b.w), "v"(e.x),
-                     "v"(e.y), "v"(e.z), "v"(e.w), "v"(m.x), "v"(m.y), "v"(m.z));
-        const BoxHit h1 = box_part(mk3(a.x, a.y, a.z), mk3(a.w, b.x, b.y), L.o, L.t_min, L.inv, L.n0, L.n1, L.n2);
-        const BoxHit h2 = box_part(mk3(b.z, b.w, e.x), mk3(e.y, e.z, e.w), L.o, L.t_min, L.inv, L.n0, L.n1, L.n2);
-        const int32_t axis = __float_as_int(m.z);
-        const bool neg = axis == 0 ? L.n0 : (axis == 1 ? L.n1 : L.n2);
-        const int32_t near_ref = __float_as_int(neg ? m.y : m.x);
-        const int32_t far_ref = __float_as_int(neg ? m.x : m.y);
-        const BoxHit hn = neg ? h2 : h1;
-        const BoxHit hf = neg ? h1 : h2;
-        const bool push = COUNT || box_pass(hf, L.t_max);
-        if (push) {
-            if (L.sp >= stk.cap) {
-                atomicOr(err, 1);
-                return true;
-            }
-            if constexpr (kSlim)
-                stack_put<SK>(stk, L.sp, far_ref);
-            else
-                stack_put<SK>(stk, L.sp, make_int2(far_ref, hf.ok ? __float_as_int(hf.lo) : kFailedLo));
+    auto entry = [&](QEnt x) {
+        if constexpr (kSlim)
+            return x.ref;
+        else
+            return i2v{ x.ref, __float_as_int(x.lo) };
+    };
+    if (SK != kStackScratch && (SK == kStackLds || L.sp + 4 <= stk.lds_entries)) {
+        // all four fit in LDS: written without branches, each over the last
+        // unless that one passed
+        BB_LDS StackEntry<ANY, false>* t = stk.lds;
+        int32_t sp = L.sp;
+        t[sp * BLOCK] = entry(x3);
+        sp += x3.ref != kNoRef;
+        t[sp * BLOCK] = entry(x2);
+        sp += x2.ref != kNoRef;
+        t[sp * BLOCK] = entry(x1);
+        sp += x1.ref != kNoRef;
+        t[sp * BLOCK] = entry(x0);
+        sp += x0.ref != kNoRef;
+        L.sp = sp;
+        return;
+    }
+    if (L.sp + 4 > stk.cap) {
+        atomicOr(err, 1);
+        L.sp = 0;
+        return;
+    }
+    const QEnt x[4] = { x3, x2, x1, x0 };
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+        if (x[k].ref != kNoRef) {
+            stack_put<SK, BLOCK>(stk, L.sp, entry(x[k]));
             ++L.sp;
         }
-        if (COUNT) c.nodes++;
-        if (box_pass(hn, L.t_max)) {
-            L.cur = near_ref;
-            return false;
+}
+
+// A lane at a leaf tests its primitives in stored order (the callbacks of
+// BVH::Intersect / IntersectAny, src/accel/bvh.cpp:299-361)
+template <bool ANY, bool COUNT, bool ALPHA>
+BB_D void leaf_test(const SceneView& S, Lane& L, TraceCount& c)
+{
+    const int32_t first = ~L.cur;
+    const float t_visit = L.t_max;
+    for (int32_t slot = first;; ++slot) {
+        const float4* tr = S.tris + 3 * size_t(slot);
+        const float4 t0 = tr[0], t1 = tr[1], t2 = tr[2];
+        // keep the three 16-byte loads together ahead of the first use
+        asm volatile("" ::"v"(t0.x), "v"(t0.y), "v"(t0.z), "v"(t1.x), "v"(t1.y), "v"(t1.z), "v"(t2.x), "v"(t2.y),
+                     "v"(t2.z), "v"(t2.w));
+        if (COUNT) c.prims++;
+        const int32_t kind = __float_as_int(t2.w);
+        float t = 0.0f, u = 0.0f, v = 0.0f;
+        // the triangle test runs on every slot so that the three loads
+        // above issue together; a sphere slot (zero edges) fails it and
+        // takes the sphere test instead
+        bool h = mt_test(xyz(t0), xyz(t1), xyz(t2), L.o, L.dn, L.l, L.t_min, L.t_max, t, u, v);
+        if ((kind & KIND_MASK) == KIND_SPHERE) {
+            u = v = 0.0f;
+            h = sphere_test(S.spheres[__float_as_int(t1.w)], L.o, L.d, L.t_min, L.t_max, t);
         }
-    } else if (L.cur != kNoRef) {
-        for (int32_t slot = ~L.cur;; ++slot) {
-            const float4 t0 = S.tris[3 * slot];
-            const float4 t1 = S.tris[3 * slot + 1];
-            const float4 t2 = S.tris[3 * slot + 2];
-            // keep the three 16-byte loads together ahead of the first use
-            asm volatile("" ::"v"(t0.x), "v"(t0.y), "v"(t0.z), "v"(t1.x), "v"(t1.y), "v"(t1.z), "v"(t2.x), "v"(t2.y),
-                         "v"(t2.z), "v"(t2.w));
-            if (COUNT) c.prims++;
-            const int32_t kind = __float_as_int(t2.w);
-            float t = 0.0f, u = 0.0f, v = 0.0f;
-            // the triangle test runs on every slot so that the three loads
-            // above issue together; a sphere slot (zero edges) fails it and
-            // takes the sphere test instead
-            bool h = mt_test(xyz(t0), xyz(t1), xyz(t2), L.o, L.dn, L.l, L.t_min, L.t_max, t, u, v);
-            if ((kind & KIND_MASK) == KIND_SPHERE) {
-                u = v = 0.0f;
-                h = sphere_test(S.spheres[__float_as_int(t1.w)], L.o, L.d, L.t_min, L.t_max, t);
+        if constexpr (!COUNT) {
+            if (h) h = leaf_visited(S, L, first, t_visit);
+        }
+        bool restarted = false;
+        if constexpr (ALPHA) { // scenes with an alpha texture only
+            if (h && (kind & kSlotAlpha)) {
+                f3 ao = L.o, ad = L.d;
+                h = alpha_chain(S, slot, ao, ad, L.t_max, t, u, v, restarted);
             }
-            bool restarted = false;
-            if constexpr (ALPHA) { // scenes with an alpha texture only
-                if (h && (kind & kSlotAlpha)) {
-                    f3 ao = L.o, ad = L.d;
-                    h = alpha_chain(S, slot, ao, ad, L.t_max, t, u, v, restarted);
-                }
+        }
+        if (h) {
+            if (COUNT) c.accepts++;
+            L.hit_slot = slot | (restarted ? kHitRestart : 0);
+            if (ANY) {
+                L.sp = 0;
+                break;
             }
-            if (h) {
-                if (COUNT) c.accepts++;
-                L.hit_slot = slot | (restarted ? kHitRestart : 0);
-                if (ANY) return true;
-                L.hit_t = t;
-                L.hit_u = u;
-                L.hit_v = v;
-                if (t <= L.t_min) return true;
-                L.t_max = t;
+            L.hit_t = t;
+            L.hit_u = u;
+            L.hit_v = v;
+            if (t <= L.t_min) {
+                L.sp = 0;
+                break;
             }
-            if (kind & kSlotLast) break;
+            L.t_max = t;
+        }
+        if (kind & kSlotLast) break;
+    }
+    L.cur = kNoRef;
+}
+
+// Takes stack entries until one is to be expanded (its deferred `lo > t_max`
+// check passes) or the stack is empty
+template <bool ANY, bool COUNT, int SK, int BLOCK>
+BB_D void take_next(Lane& L, const TraceStack<StackEntry<ANY, COUNT>>& stk, TraceCount& c)
+{
+    while (L.cur == kNoRef && L.sp > 0) {
+        --L.sp;
+        if constexpr (std::is_same<StackEntry<ANY, COUNT>, int>::value) {
+            L.cur = stack_get<SK, BLOCK>(stk, L.sp); // pushed only if it passed with this same t_max
+        } else {
+            const i2v e = stack_get<SK, BLOCK>(stk, L.sp);
+            if (COUNT) c.nodes++;
+            const bool pass = (!COUNT || e.y != kFailedLo) && !(__int_as_float(e.y) > L.t_max);
+            L.cur = pass ? e.x : kNoRef;
         }
     }
-    // take the next stack entry; its deferred `lo > t_max` check decides
-    // whether it is expanded
-    if (L.sp == 0) return true;
-    --L.sp;
-    if constexpr (kSlim) {
-        L.cur = stack_get<SK>(stk, L.sp); // pushed only if it passed with this same t_max
-    } else {
-        const int2 e = stack_get<SK>(stk, L.sp);
-        if (COUNT) c.nodes++;
-        const bool pass = (!COUNT || e.y != kFailedLo) && !(__int_as_float(e.y) > L.t_max);
-        L.cur = pass ? e.x : kNoRef;
-    }
-    return false;
 }
 
 // Queries a wave takes before the shared counter: its own part of [0, n),
@@ -530,29 +667,39 @@ BB_HD int first_chunk(int n, int waves)
 
 // Persistent traversal: a wave starts with its own part of the queries
 // (first_chunk), then takes consecutive ones from the shared counter `fetch`,
-// and hands a new query to its idle lanes once at least `refill_min` of its
-// 64 lanes are idle.  Between refill checks every lane takes STEPS traversal
-// steps.  Src provides load(index, Lane&) and finish(index, const Lane&).
-template <bool ANY, bool COUNT, int SK, bool ALPHA, int STEPS, typename Src>
+// and hands new queries to its idle lanes once at least `refill_min` of its
+// 64 lanes are idle.  In between it walks inner nodes with all lanes that are
+// at one, and tests leaves once enough lanes wait at a leaf: a ray expands
+// some ten records per leaf, so with both in every step the leaf's code ran
+// nearly each time for two or three lanes.  Each lane keeps its own order
+// of nodes and leaves.  Src provides load(index, Lane&) and
+// finish(index, const Lane&).
+template <bool ANY, bool COUNT, int SK, bool ALPHA, int BLOCK, typename Src>
 BB_D void persistent_trace(const SceneView& S, const Src& src, int n, int* fetch,
                            const TraceStack<StackEntry<ANY, COUNT>>& stk, TraceCount& c, int* err, int refill_min)
 {
     const int lane = __lane_id();
     const unsigned long long below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
-    Lane L;
-    bool active = false;
-    int id = 0;
     // the wave's reservoir of claimed queries [rb, re)
-    const int waves = gridDim.x * (blockDim.x >> 6);
-    const int wave = __builtin_amdgcn_readfirstlane(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6));
+    const int waves = gridDim.x * (BLOCK / 64);
+    const int wave = __builtin_amdgcn_readfirstlane(blockIdx.x * (BLOCK / 64) + (threadIdx.x >> 6));
     const int chunk = first_chunk(n, waves);
     const int shared = waves * chunk; // queries from here on are claimed from the counter
     int rb = min(wave * chunk, n), re = min(wave * chunk + chunk, n);
     bool more = shared < n;
+    Lane L;
+    L.cur = kNoRef; // a lane whose query is finished, or that has none (id < 0)
+    L.sp = 0;
+    int id = -1;
     for (;;) {
-        unsigned long long idle = __ballot(active ? 0 : 1);
-        if ((more || rb < re) && (__popcll(idle) >= refill_min || idle == ~0ull)) {
-            if (rb >= re) {
+        const unsigned long long idle = __ballot(L.cur == kNoRef);
+        const int n_idle = __popcll(idle);
+        if (n_idle == 64 || (n_idle >= refill_min && (more || rb < re))) {
+            if (L.cur == kNoRef && id >= 0) {
+                src.finish(id, L);
+                id = -1;
+            }
+            if (rb >= re && more) {
                 int base = 0;
                 if (lane == 0) base = atomicAdd(fetch, kReservoir);
                 const unsigned b = unsigned(shared) + unsigned(__shfl(base, 0)); // below 2^31 + waves * kReservoir
@@ -560,26 +707,34 @@ BB_D void persistent_trace(const SceneView& S, const Src& src, int n, int* fetch
                 re = n - rb > kReservoir ? rb + kReservoir : n;
                 if (re == n) more = false;
             }
-            const int rank = __popcll(idle & below);
-            const int mine = rb + rank;
-            if (!active && mine < re) {
+            if (rb >= re) {
+                if (n_idle == 64 && !more) break;
+                if (n_idle == 64) continue;
+            }
+            const int mine = rb + __popcll(idle & below);
+            if (L.cur == kNoRef && mine < re) {
                 id = mine;
                 src.load(id, L);
                 lane_root<COUNT>(S, L, c);
-                active = true;
             }
-            const int avail = re - rb, need = __popcll(idle);
-            rb += need < avail ? need : avail;
-            idle = __ballot(active ? 0 : 1);
+            rb = min(rb + n_idle, re);
         }
-        if (idle == ~0ull && !more && rb >= re) break;
-        if (idle == ~0ull) continue;
-#pragma unroll
-        for (int k = 0; k < STEPS; ++k) {
-            if (active && trace_step<ANY, COUNT, SK, ALPHA>(S, L, stk, c, err)) {
-                src.finish(id, L);
-                active = false;
+        for (;;) {
+            if (L.cur >= 0) {
+                if constexpr (COUNT)
+                    inner_expand<ANY, SK, BLOCK>(S, L, stk, c, err);
+                else
+                    quad_expand<ANY, SK, BLOCK>(S, L, stk, err);
+                take_next<ANY, COUNT, SK, BLOCK>(L, stk, c);
             }
+            const int at_node = __popcll(__ballot(L.cur >= 0));
+            const int at_leaf = __popcll(__ballot(L.cur < 0 && L.cur != kNoRef));
+            if (at_node == 0 || at_leaf >= kLeafMin || at_leaf * kLeafShare >= at_node) break;
+            if (64 - at_node - at_leaf >= refill_min && (more || rb < re)) break;
+        }
+        if (L.cur < 0 && L.cur != kNoRef) {
+            leaf_test<ANY, COUNT, ALPHA>(S, L, c);
+            take_next<ANY, COUNT, SK, BLOCK>(L, stk, c);
         }
     }
 }
@@ -699,10 +854,10 @@ template <typename E>
 BB_D TraceStack<E> make_stack(void* lds_stack, int2* gstack, int lds_entries, int cap)
 {
     TraceStack<E> t;
-    t.lds = reinterpret_cast<E*>(lds_stack) + threadIdx.x;
-    t.lstride = blockDim.x;
+    t.lds = (BB_LDS E*)(lds_stack) + threadIdx.x;
     t.gstride = gridDim.x * blockDim.x;
     t.gbl = reinterpret_cast<E*>(gstack) + blockIdx.x * blockDim.x + threadIdx.x;
+    t.priv = nullptr;
     t.lds_entries = lds_entries;
     t.cap = cap;
     return t;
@@ -713,33 +868,24 @@ template <typename E>
 BB_D TraceStack<E> make_scratch_stack(E* priv, int cap)
 {
     TraceStack<E> t;
-    t.lds = priv;
-    t.lstride = 1;
+    t.lds = nullptr;
     t.gstride = 0;
     t.gbl = nullptr;
+    t.priv = priv;
     t.lds_entries = kScratchStackEntries;
     t.cap = cap < kScratchStackEntries ? cap : kScratchStackEntries;
     return t;
 }
 
-#ifndef BB_TRACE_STEPS
-#define BB_TRACE_STEPS 2
-#endif
-constexpr int kTraceSteps = BB_TRACE_STEPS;
-#ifndef BB_SHADOW_STEPS
-#define BB_SHADOW_STEPS 2
-#endif
-constexpr int kShadowSteps = BB_SHADOW_STEPS;
-
 template <bool ANY, bool COUNT, int SK, bool ALPHA>
-__global__ __launch_bounds__(kTraceBlock) void k_trace_batch(SceneView S, BatchSrc src, int n, int* fetch,
+__global__ __launch_bounds__(kTraceBlock, ALPHA ? 1 : kTraceWaves) void k_trace_batch(SceneView S, BatchSrc src, int n, int* fetch,
                                                                int2* gstack, int lds_entries, int refill_min,
                                                                unsigned long long* counters, int* err)
 {
     extern __shared__ int2 lds_stack[];
     const auto stk = make_stack<StackEntry<ANY, COUNT>>(lds_stack, gstack, lds_entries, trace_stack_depth(S, COUNT));
     TraceCount c{ 0, 0, 0 };
-    persistent_trace<ANY, COUNT, SK, ALPHA, kTraceSteps>(S, src, n, fetch, stk, c, err, refill_min);
+    persistent_trace<ANY, COUNT, SK, ALPHA, kTraceBlock>(S, src, n, fetch, stk, c, err, refill_min);
     if (COUNT) wave_count_add(c, counters);
 }
 
@@ -937,7 +1083,7 @@ struct ShadowSrc
 // the closest-hit and shadow kernels of the bounce loop, for blocks of
 // BLOCK threads and the stack placement SK
 template <bool COUNT, int SK, bool ALPHA, int BLOCK>
-__global__ __launch_bounds__(BLOCK) void k_trace_closest(SceneView S, const int* __restrict__ n_ptr, int* fetch,
+__global__ __launch_bounds__(BLOCK, ALPHA ? 1 : kTraceWaves) void k_trace_closest(SceneView S, const int* __restrict__ n_ptr, int* fetch,
                                                          ClosestSrc src, int2* gstack, int lds_entries, int refill_min,
                                                          unsigned long long* counters, int* err)
 {
@@ -948,12 +1094,12 @@ __global__ __launch_bounds__(BLOCK) void k_trace_closest(SceneView S, const int*
                          ? make_scratch_stack<E>(priv, trace_stack_depth(S, COUNT))
                          : make_stack<E>(lds_stack, gstack, lds_entries, trace_stack_depth(S, COUNT));
     TraceCount c{ 0, 0, 0 };
-    persistent_trace<false, COUNT, SK, ALPHA, kTraceSteps>(S, src, *n_ptr, fetch, stk, c, err, refill_min);
+    persistent_trace<false, COUNT, SK, ALPHA, BLOCK>(S, src, *n_ptr, fetch, stk, c, err, refill_min);
     if (COUNT) wave_count_add(c, counters);
 }
 
 template <bool COUNT, int SK, bool ALPHA, int BLOCK>
-__global__ __launch_bounds__(BLOCK) void k_trace_shadow(SceneView S, const int* __restrict__ n_ptr, int* fetch,
+__global__ __launch_bounds__(BLOCK, ALPHA ? 1 : kTraceWaves) void k_trace_shadow(SceneView S, const int* __restrict__ n_ptr, int* fetch,
                                                         ShadowSrc src, int2* gstack, int lds_entries, int refill_min,
                                                         unsigned long long* counters, int* err)
 {
@@ -964,7 +1110,7 @@ __global__ __launch_bounds__(BLOCK) void k_trace_shadow(SceneView S, const int* 
                          ? make_scratch_stack<E>(priv, trace_stack_depth(S, COUNT))
                          : make_stack<E>(lds_stack, gstack, lds_entries, trace_stack_depth(S, COUNT));
     TraceCount c{ 0, 0, 0 };
-    persistent_trace<true, COUNT, SK, ALPHA, kShadowSteps>(S, src, *n_ptr, fetch, stk, c, err, refill_min);
+    persistent_trace<true, COUNT, SK, ALPHA, BLOCK>(S, src, *n_ptr, fetch, stk, c, err, refill_min);
     if (COUNT) wave_count_add(c, counters + 3);
 }
 
