@@ -963,7 +963,9 @@ struct PathBufs
 
 struct RenderConsts
 {
-    int32_t n_paths, npix, width, seed, max_bounces, rr_min_bounces;
+    int32_t n_paths, npix, width, height, seed, max_bounces, rr_min_bounces;
+    int32_t pass_spp;             // samples of each pixel in the pass, neighbours in the path order (order_pixel),
+                                  // or 0: path i is pixel i % npix, sample i / npix
     int32_t sample0;              // the pass's first sample relative to the call's sample_begin
     const int32_t* sample_begin;  // device copy of the call's sample_begin (set per call, read by k_raygen)
     int32_t train_stride; // cached rendering: every train_stride-th path is a training path (0: none)
@@ -999,6 +1001,23 @@ struct CacheBufs
     int32_t query_bounce, query_first, query_nee, extra, max_vertices, max_rows, max_queries;
 };
 
+// Pixel number q of the path order: down strips 8 pixels wide, row by row
+// within a strip, so that 64 pixels in a row are an 8 x 8 square.  With the
+// samples of a pixel next to each other too, the rays in flight at one time
+// come from one small part of the image, and so do their first bounces: the
+// traversal kernels read a quarter less from memory, and shading's lanes
+// meet the same material more often (24 of 64 active instead of 21).  The
+// 1080p frame of 64 spp takes 66.3 instead of 68.4 ms, the textured 801 x 451
+// frame of 8 spp 6.6 instead of 7.2, the batch of 8 scenes 64.8 instead of 66.4.
+BB_D void order_pixel(const RenderConsts& rc, int q, int& px, int& py)
+{
+    const int per_strip = 8 * rc.height;
+    const int strip = q / per_strip, r = q - strip * per_strip;
+    const int w = min(8, rc.width - 8 * strip);
+    py = w == 8 ? r >> 3 : r / w;
+    px = 8 * strip + r - py * w;
+}
+
 // UniDirectionalRayIntegrator::Render per (pixel, sample) start
 // (integrator.cpp:187-190): seed, then SampleRay(Next2D(), Next2D()) with the
 // lens sample u1 drawn first (argument evaluation of the reference's compiler),
@@ -1011,9 +1030,17 @@ __global__ __launch_bounds__(kShadeBlock) void k_raygen(GpuCamera cam, RenderCon
         P.counts[0] = rc.n_paths;
     }
     if (i >= rc.n_paths) return;
-    const int pix = i % rc.npix;
-    const int sample = *rc.sample_begin + rc.sample0 + i / rc.npix;
-    const int px = pix % rc.width, py = pix / rc.width;
+    int px, py, sample = *rc.sample_begin + rc.sample0;
+    if (rc.pass_spp > 0) {
+        const int q = i / rc.pass_spp;
+        order_pixel(rc, q, px, py);
+        sample += i - q * rc.pass_spp;
+    } else {
+        const int pix = i % rc.npix;
+        px = pix % rc.width;
+        py = pix / rc.width;
+        sample += i / rc.npix;
+    }
     uint64_t st = pcg_seed(pixel_sample_hash(px, py, rc.seed, sample));
     f2 u1;
     u1.x = pcg_float(st);
@@ -1593,24 +1620,63 @@ __global__ __launch_bounds__(kShadeBlock) void k_cache_targets(CacheBufs C, cons
 }
 
 // Film::AddSample in sample order (film.cpp:26-37); NaN/Inf samples dropped
-// (integrator.cpp:193-196).  Path i of a pass is pixel i % npix, sample i / npix.
+// (integrator.cpp:193-196).  A thread sums one pixel.  Bound by memory: when
+// a pixel's samples lie next to each other (pass_spp > 0), a wave fetches up
+// to kFilmChunk of each of its 64 pixels at a time as whole lines and hands
+// them over through LDS (1080p, 64 spp: 0.50 ms, 4.3 TB/s; each thread
+// reading its own 16-byte pieces took 2.1).
 // skip (cached renders): non-zero drops the pass (it is rendered again without the cache)
+constexpr int kFilmChunk = 8;
+
 __global__ __launch_bounds__(kShadeBlock) void k_film(RenderConsts rc, const float4* __restrict__ L, float* film_sum,
                                                        int32_t* film_count, const int32_t* skip)
 {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= rc.npix || (skip && *skip)) return;
-    float sr = film_sum[3 * p], sg = film_sum[3 * p + 1], sb = film_sum[3 * p + 2];
-    int32_t cnt = film_count[p];
-    for (int pid = p; pid < rc.n_paths; pid += rc.npix) {
-        const float4 l = L[pid];
+    __shared__ float4 s_tile[kShadeBlock / 64][64 * (kFilmChunk + 1)];
+    const int q = blockIdx.x * blockDim.x + threadIdx.x;
+    if (skip && *skip) return; // uniform over the grid
+    const bool on = q < rc.npix;
+    int p = q;
+    if (rc.pass_spp > 0 && on) {
+        int px, py;
+        order_pixel(rc, q, px, py);
+        p = py * rc.width + px;
+    }
+    float sr = 0.0f, sg = 0.0f, sb = 0.0f;
+    int32_t cnt = 0;
+    if (on) {
+        sr = film_sum[3 * p];
+        sg = film_sum[3 * p + 1];
+        sb = film_sum[3 * p + 2];
+        cnt = film_count[p];
+    }
+    auto add = [&](float4 l) {
         if (!is_nullish(mks(l.x, l.y, l.z))) {
             sr = sr + l.x;
             sg = sg + l.y;
             sb = sb + l.z;
             cnt += 1;
         }
+    };
+    if (rc.pass_spp > 1) {
+        const int lane = __lane_id(), q0 = q - lane; // the wave's first pixel
+        const int pixels = min(64, rc.npix - q0);    // <= 0 in waves past the end
+        float4* tile = s_tile[threadIdx.x >> 6];
+        for (int s0 = 0; s0 < rc.pass_spp; s0 += kFilmChunk) {
+            const int take = min(kFilmChunk, rc.pass_spp - s0);
+            for (int j = 0; j < take; ++j) {
+                const int e = j * 64 + lane, pixel = e / take, s = e - pixel * take;
+                if (pixel < pixels)
+                    tile[pixel * (kFilmChunk + 1) + s] = L[size_t(q0 + pixel) * rc.pass_spp + s0 + s];
+            }
+            __syncthreads();
+            if (on)
+                for (int s = 0; s < take; ++s) add(tile[lane * (kFilmChunk + 1) + s]);
+            __syncthreads();
+        }
+    } else if (on) {
+        for (int pid = q; pid < rc.n_paths; pid += rc.npix) add(L[pid]);
     }
+    if (!on) return;
     film_sum[3 * p] = sr;
     film_sum[3 * p + 1] = sg;
     film_sum[3 * p + 2] = sb;
@@ -2583,6 +2649,10 @@ int render_impl(BbScene* scene, const BbCameraDesc* camera, const BbRenderParams
         rc.n_paths = int32_t(n_paths);
         rc.npix = int32_t(npix);
         rc.width = camera->width;
+        rc.height = camera->height;
+        // (a cached render picks its training paths by the sample-major number; and with one sample the
+        // strips measured slower than rows: 2.30 against 2.21 ms for a 1280 x 720 preview frame)
+        rc.pass_spp = cache || k == 1 ? 0 : int32_t(k);
         rc.seed = p.seed;
         rc.sample0 = int32_t(s0);
         rc.sample_begin = P.sample_begin;

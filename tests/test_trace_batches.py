@@ -131,3 +131,22 @@ def test_scenes_at_the_margins(place):
     assert hit > 0.01
     rays["t_max"] = np.float32(1.0) if place in ("mixed", "flat") else np.float32(0.3 * np.linalg.norm(bmax - bmin))
     _same(g, o, rays, True)
+
+
+# The film at the path order's edges: strips of 8 pixels (widths 1, 7, 8, 9,
+# 65), one sample, fewer, as many and more than the film kernel takes at a
+# time (8), and several passes of unequal sample counts; every sample's value
+# is fixed by its pixel and number, so the film equals the sum of one-sample
+# films in sample order bit for bit
+@pytest.mark.gpu
+@pytest.mark.parametrize("width,height,spp,paths", [(1, 1, 3, 0), (7, 5, 8, 0), (8, 8, 2, 0), (9, 3, 9, 0), (65, 33, 17, 0),
+                                                    (65, 33, 17, 65 * 33 * 5), (16, 40, 7, 16 * 40 * 3)])
+def test_film_equals_its_samples(small, width, height, spp, paths):
+    g, _ = small
+    cam = scenes.make_camera((0.0, 2.4, 5.2), (0.0, 0.9, 0.0), 38.0, 0.0, 5.0, width, height)
+    s, c, _ = g.render(cam, scenes.render_params(spp, max_bounces=3, seed=5, wavefront_paths=paths))
+    film = g.new_film(cam)
+    for k in range(spp):
+        ws, wc, _ = g.render(cam, scenes.render_params(1, max_bounces=3, seed=5, sample_begin=k), film=film)
+    assert np.array_equal(c, wc) and np.array_equal(s.view(np.int32), ws.view(np.int32))
+    assert np.any(s > 0) or width == 1
