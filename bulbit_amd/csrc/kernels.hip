@@ -943,6 +943,11 @@ BB_D f2 filter_sample(const GpuCamera& cam, f2 u)
     return mk2((u.x * 2.0f - 1.0f) * e / 2.0f, (u.y * 2.0f - 1.0f) * e / 2.0f);
 }
 
+// What a call reads back once it is done: words 0-7 the traversal counters,
+// 8 the error flag (low half), 9-12 a cached render's results (k_cache_tally)
+constexpr int kReportWords = 16;
+constexpr int kReportErr = 8, kReportCache = 9;
+
 struct PathBufs
 {
     float4* L;     // L.rgb, eta_scale
@@ -956,8 +961,8 @@ struct PathBufs
     float4* scontrib;
     int* counts;     // [depth][4]: active paths, shadow rays, closest fetch, shadow fetch
     int2* gstack;    // traversal stack overflow, [entry][persistent thread]
-    int* err;
-    unsigned long long* counters; // [6]: closest nodes/prims/accepts, shadow nodes/prims/accepts
+    int* err;                     // in the report (kReportErr)
+    unsigned long long* counters; // the report: [6] closest nodes/prims/accepts, shadow nodes/prims/accepts first
     int* sample_begin;            // the current call's sample_begin
 };
 
@@ -1491,12 +1496,20 @@ __global__ __launch_bounds__(kShadeBlock) void k_shade(SceneView S, RenderConsts
     }
 }
 
-// the cache state at the start of a pass: queries only while the network has not diverged
-__global__ void k_cache_pass_begin(CacheBufs C)
+// the cache state at the start of a pass (queries only while the network has
+// not diverged) and of the call (first): counts and training records cleared
+__global__ void k_cache_pass_begin(CacheBufs C, int first, int n_train)
 {
-    if (threadIdx.x == 0) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n_train) C.tcount[i] = 0;
+    if (i < 4) C.counters[i] = 0;
+    if (i == 0) {
         C.state[0] = *C.diverged;
         C.state[1] = 0;
+        if (first) {
+            C.state[2] = C.state[3] = 0;
+            C.tally[0] = C.tally[1] = 0ull;
+        }
     }
 }
 
@@ -1526,17 +1539,26 @@ __global__ __launch_bounds__(kShadeBlock) void k_cache_apply(CacheBufs C, float4
 }
 
 // counts of the pass for the call's statistics: its queries and the rows its
-// `steps` optimizer steps of `batch` rows trained on
-__global__ void k_cache_tally(CacheBufs C, int steps, int batch)
+// `steps` optimizer steps of `batch` rows trained on; and the call's report
+// as of this pass: the pass dropped for a prediction that was not finite, the
+// divergence flag, the last loss, the sums of the counts
+__global__ void k_cache_tally(CacheBufs C, int steps, int batch, const float* loss, unsigned long long* report)
 {
     if (threadIdx.x != 0) return;
     C.tally[0] += (unsigned long long)min(max(C.counters[0], 0), C.max_queries);
     const int rows = min(max(C.counters[1], 0), C.max_rows);
-    if (rows == 0 || batch <= 0) return;
-    const int nb = (rows + batch - 1) / batch;
-    unsigned long long t = 0;
-    for (int s = 0; s < steps; ++s) t += (unsigned long long)min(batch, rows - (s % nb) * batch);
-    C.tally[1] += t;
+    if (rows > 0 && batch > 0) {
+        const int nb = (rows + batch - 1) / batch;
+        unsigned long long t = 0;
+        for (int s = 0; s < steps; ++s) t += (unsigned long long)min(batch, rows - (s % nb) * batch);
+        C.tally[1] += t;
+    }
+    int* r = reinterpret_cast<int*>(report + kReportCache);
+    r[0] = C.state[2];
+    r[1] = *C.diverged;
+    r[2] = __float_as_int(*loss);
+    report[kReportCache + 2] = C.tally[0];
+    report[kReportCache + 3] = C.tally[1];
 }
 
 // training rows of the pass: at each recorded vertex of a training path the
@@ -1683,21 +1705,17 @@ __global__ __launch_bounds__(kShadeBlock) void k_film(RenderConsts rc, const flo
     film_count[p] = cnt;
 }
 
-__global__ void k_zero_ints(int* p, int n)
+// The start of a call or pass in one launch: the report (when given) and the
+// queue counters cleared, and the call's sample_begin set.  One kernel for
+// each of them, and a copy back for each result, cost a render some 30 us and
+// a cached one some 100 (README scene: 0.79 to 0.76 ms at 640 x 360 x 16 spp,
+// 0.80 to 0.70 ms for a cached 1080p frame; 61 rays 62 to 46 us).
+__global__ void k_begin(unsigned long long* report, int* counts, int n_counts, int* sample_begin, int value)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = 0;
-}
-
-__global__ void k_set_int(int* p, int v)
-{
-    if (blockIdx.x == 0 && threadIdx.x == 0) *p = v;
-}
-
-__global__ void k_zero_u64(unsigned long long* p, int n)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = 0ull;
+    if (report && i < kReportWords) report[i] = 0ull;
+    if (i < n_counts) counts[i] = 0;
+    if (sample_begin && i == 0) *sample_begin = value;
 }
 
 } // namespace bb
@@ -1860,13 +1878,14 @@ bool ensure_workspace(Workspace& w, size_t paths, int depth_slots)
               dalloc(w, &P.flags, paths) && dalloc(w, &P.queue[0], paths) && dalloc(w, &P.queue[1], paths) &&
               dalloc(w, &P.ray[0], 2 * paths) && dalloc(w, &P.ray[1], 2 * paths) && dalloc(w, &P.hit, paths) &&
               dalloc(w, &P.sray, 2 * paths) && dalloc(w, &P.scontrib, paths) &&
-              dalloc(w, &P.counts, size_t(4) * (depth_slots + 2)) && dalloc(w, &P.err, 4) && dalloc(w, &P.counters, 8) &&
+              dalloc(w, &P.counts, size_t(4) * (depth_slots + 2)) && dalloc(w, &P.counters, kReportWords) &&
               dalloc(w, &P.sample_begin, 1);
     if (!ok) {
         for (void* p : w.allocs) hipFree(p);
         w.allocs.clear();
         return false;
     }
+    P.err = reinterpret_cast<int*>(P.counters + kReportErr);
     w.capacity = paths;
     w.max_depth_slots = depth_slots;
     w.P.gstack = reinterpret_cast<int2*>(w.gstack);
@@ -2159,9 +2178,8 @@ TracePlan trace_plan(const SceneView& V, int32_t n_rays, int32_t any_hit, bool c
 // The device memory a traversal batch uses beyond its rays and hits
 struct TraceScratch
 {
-    int* err;                     // 1: a traversal stack overflowed
-    int* counts;                  // [4]: the work-queue fetch counter at [0]
-    unsigned long long* counters; // [8]: nodes, prims, accepts
+    int* counts;                // [4]: the work-queue fetch counter at [0]
+    unsigned long long* report; // [kReportWords]: nodes, prims, accepts; the error flag (1: a traversal stack overflowed)
     int2* gstack;                 // the stack's overflow area, plan.overflow_per_lane entries per lane
 };
 
@@ -2169,20 +2187,19 @@ struct TraceScratch
 int trace_run(const char* who, const SceneView& V, const BbRay* rays, int32_t n_rays, int32_t any_hit, BbHit* hits,
               BbTraceCounters* counters, hipStream_t st, const TracePlan& t, const TraceScratch& s)
 {
-    hipLaunchKernelGGL(k_zero_ints, dim3(1), dim3(64), 0, st, s.err, 1);
-    hipLaunchKernelGGL(k_zero_ints, dim3(1), dim3(64), 0, st, s.counts, 4);
-    hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(64), 0, st, s.counters, 8);
+    int* err_dev = reinterpret_cast<int*>(s.report + kReportErr);
+    hipLaunchKernelGGL(k_begin, dim3(1), dim3(64), 0, st, s.report, s.counts, 4, (int*)nullptr, 0);
     if (n_rays > 0) {
         BatchSrc src{ reinterpret_cast<const float4*>(rays), reinterpret_cast<int4*>(hits), V.tris, any_hit };
         hipLaunchKernelGGL(t.kfn, dim3(t.grid), dim3(kTraceBlock), t.lds, st, V, src, n_rays, s.counts, s.gstack,
-                           t.lds_entries, 48, s.counters, s.err);
+                           t.lds_entries, 48, s.report, err_dev);
         HIP_OK(hipGetLastError());
     }
     int err = 0;
-    unsigned long long c[8] = { 0 };
-    HIP_OK(hipMemcpyAsync(&err, s.err, sizeof(int), hipMemcpyDeviceToHost, st));
-    HIP_OK(hipMemcpyAsync(c, s.counters, sizeof(c), hipMemcpyDeviceToHost, st));
+    unsigned long long c[kReportWords] = { 0 };
+    HIP_OK(hipMemcpyAsync(c, s.report, sizeof(c), hipMemcpyDeviceToHost, st));
     HIP_OK(hipStreamSynchronize(st));
+    memcpy(&err, &c[kReportErr], sizeof(int));
     if (err) {
         bb::set_error("%s: traversal stack overflow", who);
         return BBGPU_ERR_DEVICE;
@@ -2197,8 +2214,8 @@ int trace_run(const char* who, const SceneView& V, const BbRay* rays, int32_t n_
 }
 
 // Scratch of bbgpu_trace_noalloc, one copy per device (it lives as long as
-// the process): a 256-byte header (counters at 0, the error flag at 64, the
-// work-queue counts at 128), then the traversal stacks' overflow area.  Host
+// the process): a 256-byte header (the report at 0, the work-queue
+// counts at 128), then the traversal stacks' overflow area.  Host
 // code never passes `scratch` itself to a kernel (its host-side name is not a
 // device address); it uses the address hipGetSymbolAddress returns for the
 // current device.
@@ -2275,7 +2292,7 @@ int bbgpu_trace(BbScene* scene, const BbRay* rays_dev, int32_t n_rays, int32_t a
         }
         if (host_hits) hits = reinterpret_cast<BbHit*>(stage + rb);
     }
-    const TraceScratch s{ P.err, P.counts, P.counters, P.gstack };
+    const TraceScratch s{ P.counts, P.counters, P.gstack };
     const int r = trace_run("bbgpu_trace", V, rays, n_rays, any_hit, hits, counters, st, t, s);
     if (r == BBGPU_OK && host_hits)
         HIP_OK(hipMemcpy(hits_dev, hits, sizeof(BbHit) * size_t(n_rays), hipMemcpyDeviceToHost));
@@ -2313,8 +2330,8 @@ int bbgpu_trace_noalloc(BbScene* scene, const BbRay* rays_dev, int32_t n_rays, i
         }
         t.grid = int(std::min<size_t>(size_t(t.grid), fit));
     }
-    const TraceScratch s{ reinterpret_cast<int*>(base + 64), reinterpret_cast<int*>(base + 128),
-                          reinterpret_cast<unsigned long long*>(base),
+    static_assert(sizeof(unsigned long long) * kReportWords <= 128, "the report fits before the counts");
+    const TraceScratch s{ reinterpret_cast<int*>(base + 128), reinterpret_cast<unsigned long long*>(base),
                           reinterpret_cast<int2*>(base + kNoAllocHeaderBytes) };
     return trace_run("bbgpu_trace_noalloc", V, rays_dev, n_rays, any_hit, hits_dev, counters, (hipStream_t)stream, t, s);
 }
@@ -2578,8 +2595,6 @@ int render_impl(BbScene* scene, const BbCameraDesc* camera, const BbRenderParams
         C->extra = std::max(0, cache->cp.train_extra_bounces);
         C->diverged = nrc_status(cache->nrc);
         if (cache->stats) memset(cache->stats, 0, sizeof(*cache->stats));
-        hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(64), 0, st, C->tally, 2);
-        hipLaunchKernelGGL(k_zero_ints, dim3(1), dim3(64), 0, st, C->state, 4);
     }
     CacheBufs Cv{};
     if (C) Cv = *C;
@@ -2598,13 +2613,14 @@ int render_impl(BbScene* scene, const BbCameraDesc* camera, const BbRenderParams
     hipEvent_t t_begin = nullptr;
     if (timed) t_begin = mark();
     hipEvent_t t_begin_all = (cache && cache->stats) ? mark() : nullptr;
-    // the one value that differs between calls that share a captured graph
-    hipLaunchKernelGGL(k_set_int, dim3(1), dim3(64), 0, st, P.sample_begin, p.sample_begin);
-
     // Graph mode: the launch sequence below has no host synchronization when
     // neither stats nor the cache are on; it is captured once on the scene's
     // capture stream and replayed on the caller's stream
     const bool use_graph = p.graph != 0 && !timed && !cache;
+    // the one value that differs between calls that share a captured graph
+    if (use_graph)
+        hipLaunchKernelGGL(k_begin, dim3(1), dim3(64), 0, st, (unsigned long long*)nullptr, (int*)nullptr, 0,
+                           P.sample_begin, p.sample_begin);
     GraphEntry* graph = nullptr;
     bool capturing = false;
     std::vector<unsigned char> key;
@@ -2638,10 +2654,6 @@ int render_impl(BbScene* scene, const BbCameraDesc* camera, const BbRenderParams
     int64_t paths_total = 0;
     int pass = 0;
     const bool replay = graph != nullptr; // a captured graph stands in for the launches below
-    if (!replay) {
-        hipLaunchKernelGGL(k_zero_ints, dim3(1), dim3(64), 0, ls, P.err, 1);
-        hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(64), 0, ls, P.counters, 8);
-    }
     for (long long s0 = 0; !replay && s0 < p.spp; s0 += per_pass) {
         const long long k = std::min<long long>(per_pass, p.spp - s0);
         const long long n_paths = k * npix;
@@ -2662,12 +2674,12 @@ int render_impl(BbScene* scene, const BbCameraDesc* camera, const BbRenderParams
         rc.train_stride = stride;
         paths_total += n_paths;
         hipEvent_t a = timed ? mark() : nullptr;
-        hipLaunchKernelGGL(k_zero_ints, dim3((nslots + 255) / 256), dim3(256), 0, ls, P.counts, nslots);
+        hipLaunchKernelGGL(k_begin, dim3((nslots + 255) / 256), dim3(256), 0, ls, s0 == 0 ? P.counters : nullptr,
+                           P.counts, nslots, s0 == 0 && !use_graph ? P.sample_begin : nullptr, p.sample_begin);
         const int n_train = cache ? int((n_paths + stride - 1) / stride) : 0;
         if (cache) {
-            hipLaunchKernelGGL(k_cache_pass_begin, dim3(1), dim3(64), 0, ls, Cv);
-            hipLaunchKernelGGL(k_zero_ints, dim3(1), dim3(64), 0, ls, Cv.counters, 4);
-            hipLaunchKernelGGL(k_zero_ints, dim3((n_train + 255) / 256), dim3(256), 0, ls, Cv.tcount, n_train);
+            hipLaunchKernelGGL(k_cache_pass_begin, dim3((n_train + 255) / 256), dim3(256), 0, ls, Cv, s0 == 0 ? 1 : 0,
+                               n_train);
         }
         hipLaunchKernelGGL(k_raygen, dim3(unsigned((n_paths + kShadeBlock - 1) / kShadeBlock)), dim3(kShadeBlock), 0, ls,
                            cam, rc, P);
@@ -2727,7 +2739,8 @@ int render_impl(BbScene* scene, const BbCameraDesc* camera, const BbRenderParams
                 if (rt != BBGPU_OK) return rt;
             }
             hipEvent_t q3 = cache_timed ? mark() : nullptr;
-            hipLaunchKernelGGL(k_cache_tally, dim3(1), dim3(64), 0, st, Cv, cache->cp.train_steps, batch);
+            hipLaunchKernelGGL(k_cache_tally, dim3(1), dim3(64), 0, st, Cv, cache->cp.train_steps, batch,
+                               nrc_loss(cache->nrc), P.counters);
             if (cache_timed) {
                 spans.push_back({ q0, q1, 3 });
                 spans.push_back({ q1, q2, 5 });
@@ -2770,35 +2783,40 @@ int render_impl(BbScene* scene, const BbCameraDesc* camera, const BbRenderParams
         graph = &x->graphs.back();
     }
     if (graph) HIP_OK(hipGraphLaunch(graph->exec, st));
+    unsigned long long c[kReportWords] = { 0 };
+    hipEvent_t t_end = nullptr;
     if (cache) {
-        // one synchronization per call: the pass dropped for non-finite
-        // predictions (rendered again without the cache, into the same film),
-        // the divergence flag and the statistics
-        int stv[4] = { 0, 0, 0, 0 };
-        int flag = 0;
-        unsigned long long tally[2] = { 0, 0 };
-        float loss = 0.0f;
-        HIP_OK(hipMemcpyAsync(stv, Cv.state, sizeof(stv), hipMemcpyDeviceToHost, st));
-        HIP_OK(hipMemcpyAsync(&flag, Cv.diverged, sizeof(int), hipMemcpyDeviceToHost, st));
-        HIP_OK(hipMemcpyAsync(tally, Cv.tally, sizeof(tally), hipMemcpyDeviceToHost, st));
-        HIP_OK(hipMemcpyAsync(&loss, nrc_loss(cache->nrc), sizeof(float), hipMemcpyDeviceToHost, st));
+        // one synchronization per call: the report tells of a pass dropped for
+        // non-finite predictions (rendered again without the cache, into the
+        // same film), the divergence flag and the statistics
+        if (cache->stats) t_end = mark();
+        HIP_OK(hipMemcpyAsync(c, P.counters, sizeof(c), hipMemcpyDeviceToHost, st));
         HIP_OK(hipStreamSynchronize(st));
+        int words[3]; // the dropped pass + 1, the flag, the loss
+        memcpy(words, &c[kReportCache], sizeof(words));
+        const int dropped = words[0], flag = words[1];
+        float loss;
+        memcpy(&loss, &words[2], sizeof(float));
         nrc_note_diverged(cache->nrc, flag != 0);
-        if (stv[2] > 0) {
-            const long long s0 = (long long)(stv[2] - 1) * per_pass;
+        if (dropped > 0) {
+            const long long s0 = (long long)(dropped - 1) * per_pass;
             BbRenderParams rp = p;
             rp.sample_begin = p.sample_begin + int32_t(s0);
             rp.spp = int32_t(std::min<long long>(per_pass, p.spp - s0));
             rp.graph = 0;
             const int rr = render_impl(scene, camera, &rp, film_sum_dev, film_count_dev, stream, nullptr, 0, nullptr);
             if (rr != BBGPU_OK) return rr;
+            if (cache->stats) {
+                t_end = mark();
+                HIP_OK(hipStreamSynchronize(st));
+            }
         }
         if (cache->stats) {
-            cache->stats->queries = int64_t(tally[0]);
-            cache->stats->train_rows = int64_t(tally[1]);
+            cache->stats->queries = int64_t(c[kReportCache + 2]);
+            cache->stats->train_rows = int64_t(c[kReportCache + 3]);
             cache->stats->loss = loss;
             cache->stats->diverged = flag != 0 ? 1 : 0;
-            cache->stats->passes_redone = stv[2] > 0 ? 1 : 0;
+            cache->stats->passes_redone = dropped > 0 ? 1 : 0;
             for (const Span& sp : spans) {
                 float d = 0.0f;
                 hipEventElapsedTime(&d, sp.a, sp.b);
@@ -2808,17 +2826,16 @@ int render_impl(BbScene* scene, const BbCameraDesc* camera, const BbRenderParams
             }
         }
     }
-    hipEvent_t t_end = (timed || (cache && cache->stats)) ? mark() : nullptr;
+    if (timed) t_end = mark();
     if (host_film) {
         HIP_OK(hipMemcpyAsync(film_sum_user, film_sum_dev, sum_bytes, hipMemcpyDeviceToHost, st));
         HIP_OK(hipMemcpyAsync(film_count_user, film_count_dev, count_bytes, hipMemcpyDeviceToHost, st));
     }
     if (!wait && !timed && !host_film && !cache) return BBGPU_OK;
+    if (!cache) HIP_OK(hipMemcpyAsync(c, P.counters, sizeof(c), hipMemcpyDeviceToHost, st));
+    if (!cache || host_film) HIP_OK(hipStreamSynchronize(st));
     int err = 0;
-    unsigned long long c[8] = { 0 };
-    HIP_OK(hipMemcpyAsync(&err, P.err, sizeof(int), hipMemcpyDeviceToHost, st));
-    HIP_OK(hipMemcpyAsync(c, P.counters, sizeof(c), hipMemcpyDeviceToHost, st));
-    HIP_OK(hipStreamSynchronize(st));
+    memcpy(&err, &c[kReportErr], sizeof(int));
     if (err) {
         bb::set_error("bbgpu_render: traversal stack overflow");
         return BBGPU_ERR_DEVICE;
