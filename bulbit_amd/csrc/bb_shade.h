@@ -9,8 +9,9 @@
 //   include/bulbit/bsdf.h:75-125                             BSDF wrapper
 //   src/light/{spot_light,uniform_infinite_light,diffuse_area_light}.cpp
 //
-// Transcendentals: sin, cos and pow are evaluated in double precision and
-// rounded once to float, which reproduces a correctly rounded float result;
+// Transcendentals: sin, cos (bb_trig.h) and pow are evaluated in double
+// precision and rounded once to float, a correctly rounded float result in
+// practice;
 // the reference's glibc sinf/cosf agree with it except in ~1% of arguments
 // (by one ulp).  Division and sqrt are IEEE (correctly rounded) on gfx950
 // with the library's compile flags.
@@ -18,12 +19,11 @@
 
 #include "bb_scene.h"
 #include "bb_texcoord.h"
+#include "bb_trig.h"
 
 namespace bb
 {
 
-BB_D float dsin(float x) { return (float)::sin((double)x); }
-BB_D float dcos(float x) { return (float)::cos((double)x); }
 BB_D float dpow(float x, float y) { return (float)::pow((double)x, (double)y); }
 BB_D float dacos(float x) { return (float)::acos((double)x); }
 
@@ -42,7 +42,9 @@ BB_D f2 sample_concentric(f2 u)
         r = uo.y;
         theta = (kPi / 2.0f) - (kPi / 4.0f) * (uo.x / uo.y);
     }
-    return mk2(dcos(theta) * r, dsin(theta) * r);
+    float sn, cs;
+    sincos_small(theta, sn, cs);
+    return mk2(cs * r, sn * r);
 }
 
 // SampleUniformSphere, sampling.h:64-74
@@ -51,7 +53,9 @@ BB_D f3 sample_uniform_sphere(f2 u)
     float z = 1.0f - 2.0f * u.x;
     float r = sqrtf(fmaxf(0.0f, 1.0f - z * z));
     float phi = kTwoPi * u.y;
-    return mk3(r * dcos(phi), r * dsin(phi), z);
+    float sn, cs;
+    sincos_small(phi, sn, cs);
+    return mk3(r * cs, r * sn, z);
 }
 
 // SampleCosineHemisphere (Malley), sampling.h:151-169
@@ -193,8 +197,10 @@ BB_D f3 ggx_sample_wm(ggx m, f3 wo, f2 u)
     float phi = kTwoPi * u.x;
     float z = fmaf((1.0f - u.y), (1.0f + wo_std.z), -wo_std.z);
     float sin_t = sqrtf(clampf_(1.0f - z * z, 0.0f, 1.0f));
-    float x = sin_t * dcos(phi);
-    float y = sin_t * dsin(phi);
+    float sn, cs;
+    sincos_small(phi, sn, cs);
+    float x = sin_t * cs;
+    float y = sin_t * sn;
     f3 h = mk3(x, y, z) + wo_std;
     return normalize(mk3(h.x * m.ax, h.y * m.ay, h.z));
 }
@@ -439,8 +445,10 @@ BB_D f3 eon_cltc_sample(f3 wo, float r, float u1, float u2, float& pdf)
     eon_ltc(wo.z, r, a, b, c, d);
     const float R = sqrtf(u1);
     const float phi = kTwoPi * u2;
-    float x = R * dcos(phi);
-    const float y = R * dsin(phi);
+    float sn, cs;
+    sincos_small(phi, sn, cs);
+    float x = R * cs;
+    const float y = R * sn;
     const float vz = 1.0f / sqrtf(d * d + 1.0f);
     const float s = 0.5f * (1.0f + vz);
     x = -(sqrtf(1.0f - y * y) * (1.0f - s) + x * s); // -Lerp(sqrt(1 - y^2), x, s)
@@ -500,7 +508,9 @@ BB_D bool eon_sample(const bxdf& b, f3 wo, float u0, f2 u12, bsample& out)
         const float z = u12.x;
         const float rr = sqrtf(fmaxf(0.0f, 1.0f - z * z));
         const float phi = kTwoPi * u12.y;
-        wi = mk3(rr * dcos(phi), rr * dsin(phi), z);
+        float sn, cs;
+        sincos_small(phi, sn, cs);
+        wi = mk3(rr * cs, rr * sn, z);
         pdf_c = eon_cltc_pdf(wo, wi, r);
     } else {
         wi = eon_cltc_sample(wo, r, u12.x, u12.y, pdf_c);
@@ -653,7 +663,7 @@ BB_D float dielectric_pdf(const bxdf& b, f3 wo, f3 wi)
 
 // Metallic-roughness, metallic_roughness_bxdf.cpp:8-80, bxdfs.h:466-489
 BB_D spec mr_F0(const bxdf& b) { return mks(0.04f) * (1.0f - b.metallic) + b.color * b.metallic; }
-BB_D spec mr_schlick(spec f0, float c) { return f0 + (mks(1.0f) - f0) * dpow(1.0f - c, 5.0f); }
+BB_D spec mr_schlick(spec f0, float c) { return f0 + (mks(1.0f) - f0) * pow5(1.0f - c); }
 BB_D spec mr_f(const bxdf& b, f3 wo, f3 wi)
 {
     if (!same_hemisphere(wo, wi)) return mks(0.0f);

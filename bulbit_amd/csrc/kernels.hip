@@ -1244,9 +1244,20 @@ BB_D void cache_features(const CacheBufs& C, const GpuMaterial& m, f3 p, f3 wo, 
     r[13] = r[14] = r[15] = 0.0f;
 }
 
+constexpr int kKindsLcd = (1 << MK_LAMBERT) | (1 << MK_CONDUCTOR) | (1 << MK_DIELECTRIC);
+constexpr int kKindsMr = (1 << MK_METALLIC_ROUGHNESS) | (1 << MK_LAMBERT);
+
+// Waves per SIMD that shading with every BxDF is built for: left alone the
+// compiler takes 297 VGPRs for the textured kernel and one wave fits (801 x
+// 451 frame of 8 spp, textures in every slot: 6.5 ms; bound to three, with
+// some spills, 5.7; to four 6.0).  The kernels for fewer kinds need 154 and
+// 155 and are best left alone (Lambertian + conductor + dielectric bound to
+// four: the 1080p frame of 64 spp 67.4 instead of 65.8 ms).
+constexpr int kShadeWavesAll = 3;
+
 // KM: the BxDF kinds compiled in (the scene's materials' kinds, or all)
 template <bool CACHE, bool TEX, int KM>
-__global__ __launch_bounds__(kShadeBlock) void k_shade(SceneView S, RenderConsts rc, PathBufs P, int depth, CacheBufs C)
+__global__ __launch_bounds__(kShadeBlock, KM == kAllKinds ? kShadeWavesAll : 1) void k_shade(SceneView S, RenderConsts rc, PathBufs P, int depth, CacheBufs C)
 {
     const int in = depth & 1, out = in ^ 1;
     const int n = P.counts[4 * depth];
@@ -2051,8 +2062,6 @@ int trace_grid(const void* kernel, size_t lds_bytes, int block = kTraceBlock)
 // textures, and the BxDF code of the scene's material kinds only (two
 // common sets: Lambertian + conductor + dielectric, and metallic-roughness +
 // Lambertian), so the common kernels need fewer registers
-constexpr int kKindsLcd = (1 << MK_LAMBERT) | (1 << MK_CONDUCTOR) | (1 << MK_DIELECTRIC);
-constexpr int kKindsMr = (1 << MK_METALLIC_ROUGHNESS) | (1 << MK_LAMBERT);
 using ShadeKernel = void (*)(SceneView, RenderConsts, PathBufs, int, CacheBufs);
 
 template <bool CACHE>
