@@ -531,12 +531,12 @@ bool textures_to_gpu(const BbSceneDesc& d, std::vector<GpuTexture>& out, std::ve
     return true;
 }
 
-// fn(i) for i in [0, n), on several threads from 2^15 items up; fn(i) writes
+// fn(i) for i in [0, n), on several threads from 2^14 items up; fn(i) writes
 // what belongs to i alone
 template <typename F>
 void for_each_index(int64_t n, F fn)
 {
-    const int64_t threads = std::min<int64_t>({ n >> 15, 8, int64_t(std::max(1u, std::thread::hardware_concurrency())) });
+    const int64_t threads = std::min<int64_t>({ n >> 13, 8, int64_t(std::max(1u, std::thread::hardware_concurrency())) });
     auto part = [&](int64_t k, int64_t of) {
         for (int64_t i = n * k / of; i < n * (k + 1) / of; ++i) fn(i);
     };
