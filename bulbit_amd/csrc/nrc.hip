@@ -19,7 +19,7 @@
 // training step of the 64-wide network permute the k slots (frag_feature).
 //
 // Training step of the 128-wide network: the forward pass saves every
-// layer's bf16 input per chunk of 64 rows, feature-major; k_mlp_dz runs the
+// layer's bf16 input per chunk of kRows rows, feature-major; k_mlp_dz runs the
 // gradient chain dz_{l-1} = (dz_l W_l^T) masked by h_l > 0 per chunk and
 // saves each dz_l, also feature-major; k_mlp_dw forms dW_l = h_l^T dz_l as a
 // GEMM over the rows (whose operands are exactly those saved layouts), split
@@ -54,8 +54,14 @@ namespace bb
 constexpr int kIn = 80;      // encoded input width (74 used)
 constexpr int kOutCols = 16; // output columns (3 used)
 constexpr int kRawStride = 16;
-constexpr int kRows = 64;    // rows per wave per chunk (4 row tiles of 16)
+// Rows per wave and chunk of the wide network's training step.  A step of
+// 65,536 rows is as many chunks as the chip has SIMDs at 64 rows, so every
+// latency showed; with 32 two waves share a SIMD (forward / gradient chain /
+// dW kernels 45 / 61 / 55 -> 37 / 54 / 39 us, four steps 745 -> 620 us).
+constexpr int kRows = 32;
+constexpr int kTiles = kRows / 16; // row tiles of a chunk
 constexpr int kNrcBlock = 256;
+constexpr int kPad = 8;      // bf16 values added to a row of a tile in LDS
 
 // One network shape.  Weight matrices: W_0 [kIn][W], W_1..W_{L-1} [W][W],
 // W_L [W][kOutCols]; fp32 master copies k-major ([k][n]).
@@ -67,12 +73,14 @@ struct Net
     static constexpr int n(int l) { return l == L ? kOutCols : W; }
     static constexpr int off(int l) { return l == 0 ? 0 : off(l - 1) + k(l - 1) * n(l - 1); }
     static constexpr int params = off(L + 1);
-    static constexpr int max_layer = (kIn * W > W * W ? kIn * W : W * W);
-    // row stride (bf16) of a wave's activation tile in the forward pass
-    static constexpr int ld = W > kIn ? W : kIn;
-    // the whole bf16 network stays in LDS when it fits beside four
-    // activation tiles; otherwise each layer is staged in turn
-    static constexpr bool resident = params * 2 + 4 * kRows * ld * 2 <= 96 * 1024;
+    // row strides (bf16) of the tiles in LDS of the training step's forward
+    // pass (a wave's activations, a layer's staged weights) and gradient chain:
+    // eight more than the row, since rows of 256 bytes start in one bank and
+    // the operand reads, 16 rows at a time, met 16 deep (forward kernel over
+    // 65,536 rows 53 -> 45 us)
+    static constexpr int ld = (W > kIn ? W : kIn) + kPad;
+    static constexpr int ldz = W + kPad;
+    static constexpr int max_layer = W * (W > kIn ? W + kPad : kIn + kPad);
     // Layer inputs saved by the training forward pass, per chunk of kRows
     // rows, feature-major ([feature][row in chunk]): h_0 (kIn features), then
     // h_1..h_L (W each).  Eight consecutive rows of one feature are one 16-byte
@@ -87,6 +95,7 @@ struct Net
     // 80 x 64 blocks (5 x 4 tiles), the hidden layers in 64 x 64 blocks,
     // the output layer in 64 x 16 blocks
     static constexpr int groups = W / 64 + (L - 1) * (W / 64) * (W / 64) + W / 64;
+    static constexpr int dw_waves = W / 64 > 1 ? (W / 64) * (W / 64) : 2; // waves of a dW block
     // The query kernel's weights: per layer, W_l^T cut into the A-operand
     // fragments of v_mfma_f32_16x16x32_bf16 (16 output features x 32 input
     // features, K padded to a multiple of 32), fragment (l, k-step, m-tile)
@@ -240,22 +249,22 @@ BB_D f4v mfma32(s8v a, s8v b, f4v c)
 }
 
 // one layer for a wave's kRows rows: act [kRows][ld_in] (bf16, LDS) times
-// W_l (WT: [n][k] bf16, LDS) -> acc[row tile][col tile]
+// W_l (WT: [n][k] bf16, LDS, rows K + kPad apart) -> acc[row tile][col tile]
 template <int K, int N>
-BB_D void layer_forward(const uint16_t* act, int ld_in, const uint16_t* WT, f4v (&acc)[4][N / 16], int lane)
+BB_D void layer_forward(const uint16_t* act, int ld_in, const uint16_t* WT, f4v (&acc)[kTiles][N / 16], int lane)
 {
     const int r16 = lane & 15, q = lane >> 4;
 #pragma unroll
-    for (int rt = 0; rt < 4; ++rt)
+    for (int rt = 0; rt < kTiles; ++rt)
 #pragma unroll
         for (int ct = 0; ct < N / 16; ++ct) acc[rt][ct] = f4v{ 0.0f, 0.0f, 0.0f, 0.0f };
 #pragma unroll
     for (int kk = 0; kk < K / 32; ++kk) {
         s8v b[N / 16];
 #pragma unroll
-        for (int ct = 0; ct < N / 16; ++ct) b[ct] = load8(WT + (ct * 16 + r16) * K + kk * 32 + q * 8);
+        for (int ct = 0; ct < N / 16; ++ct) b[ct] = load8(WT + (ct * 16 + r16) * (K + kPad) + kk * 32 + q * 8);
 #pragma unroll
-        for (int rt = 0; rt < 4; ++rt) {
+        for (int rt = 0; rt < kTiles; ++rt) {
             const s8v a = load8(act + (rt * 16 + r16) * ld_in + kk * 32 + q * 8);
 #pragma unroll
             for (int ct = 0; ct < N / 16; ++ct) acc[rt][ct] = mfma32(a, b[ct], acc[rt][ct]);
@@ -265,9 +274,9 @@ BB_D void layer_forward(const uint16_t* act, int ld_in, const uint16_t* WT, f4v 
         constexpr int k0 = K - 16;
         s4 b[N / 16];
 #pragma unroll
-        for (int ct = 0; ct < N / 16; ++ct) b[ct] = load4(WT + (ct * 16 + r16) * K + k0 + q * 4);
+        for (int ct = 0; ct < N / 16; ++ct) b[ct] = load4(WT + (ct * 16 + r16) * (K + kPad) + k0 + q * 4);
 #pragma unroll
-        for (int rt = 0; rt < 4; ++rt) {
+        for (int rt = 0; rt < kTiles; ++rt) {
             const s4 a = load4(act + (rt * 16 + r16) * ld_in + k0 + q * 4);
 #pragma unroll
             for (int ct = 0; ct < N / 16; ++ct) acc[rt][ct] = mfma(a, b[ct], acc[rt][ct]);
@@ -281,6 +290,16 @@ BB_D void stage16(uint16_t* dst, const uint16_t* src, int count)
 {
     for (int i = threadIdx.x; i < count / 8; i += blockDim.x)
         reinterpret_cast<uint4*>(dst)[i] = reinterpret_cast<const uint4*>(src)[i];
+}
+
+// rows x k bf16 values (k a multiple of 8) into LDS rows of k + kPad
+BB_D void stage_rows(uint16_t* dst, const uint16_t* src, int rows, int k)
+{
+    const int per = k / 8;
+    for (int i = threadIdx.x; i < rows * per; i += blockDim.x) {
+        const int r = i / per;
+        *reinterpret_cast<uint4*>(dst + r * (k + kPad) + (i - r * per) * 8) = reinterpret_cast<const uint4*>(src)[i];
+    }
 }
 
 // ---------------------------------------------------------------- forward
@@ -303,13 +322,9 @@ __global__ __launch_bounds__(kNrcBlock) void k_mlp_forward(const float* __restri
     int off = 0, n = 0;
     span_rows(span, off, n);
     raw += size_t(off) * kRawStride;
-    __shared__ __align__(16) uint16_t sW[NT::resident ? NT::params : NT::max_layer];
+    __shared__ __align__(16) uint16_t sW[NT::max_layer];
     __shared__ __align__(16) uint16_t sAct[kNrcBlock / 64][kRows * LD];
-    static_assert(NT::params % 8 == 0 && NT::max_layer % 8 == 0, "weights staged 16 bytes at a time");
-    if constexpr (NT::resident) {
-        stage16(sW, Wt.WT, NT::params);
-        __syncthreads();
-    }
+    static_assert(kIn % 8 == 0 && W % 8 == 0, "weights staged 16 bytes at a time");
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     uint16_t* act = sAct[wave];
     const int r16 = lane & 15, q = lane >> 4;
@@ -319,34 +334,34 @@ __global__ __launch_bounds__(kNrcBlock) void k_mlp_forward(const float* __restri
         const bool active = ch < chunks;
         const int row0 = ch * kRows;
         if (active) {
-            // each lane encodes its row straight into the wave's LDS rows
+            // a lane encodes a row straight into the wave's LDS rows
             const int row = row0 + lane;
             uint16_t* e = act + lane * LD;
-            if (row < n)
-                encode_row(raw + size_t(row) * kRawStride, e);
-            else
-                for (int i = 0; i < kIn; ++i) e[i] = 0;
-            if (SAVE) // every row of the chunk, zeros beyond n
-                for (int i = 0; i < kIn; ++i) acts[size_t(ch) * NT::chunk_acts + NT::act_off(0) + i * kRows + lane] = e[i];
+            if (lane < kRows) {
+                if (row < n)
+                    encode_row(raw + size_t(row) * kRawStride, e);
+                else
+                    for (int i = 0; i < kIn; ++i) e[i] = 0;
+                if (SAVE) // every row of the chunk, zeros beyond n
+                    for (int i = 0; i < kIn; ++i)
+                        acts[size_t(ch) * NT::chunk_acts + NT::act_off(0) + i * kRows + lane] = e[i];
+            }
         }
         // hidden layers in a rolled loop (one copy of the code: small kernels
         // stay in the instruction cache)
 #pragma unroll 1
         for (int l = 0; l < L; ++l) {
-            const uint16_t* Wl = sW + (NT::resident ? NT::off(l) : 0);
-            if constexpr (!NT::resident) {
-                __syncthreads(); // every wave is done with the previous layer's weights
-                stage16(sW, Wt.WT + NT::off(l), NT::k(l) * NT::n(l));
-                __syncthreads();
-            }
+            __syncthreads(); // every wave is done with the previous layer's weights
+            stage_rows(sW, Wt.WT + NT::off(l), NT::n(l), NT::k(l));
+            __syncthreads();
             if (!active) continue;
-            f4v acc[4][W / 16];
+            f4v acc[kTiles][W / 16];
             if (l == 0)
-                layer_forward<kIn, W>(act, LD, Wl, acc, lane);
+                layer_forward<kIn, W>(act, LD, sW, acc, lane);
             else
-                layer_forward<W, W>(act, LD, Wl, acc, lane);
+                layer_forward<W, W>(act, LD, sW, acc, lane);
 #pragma unroll
-            for (int rt = 0; rt < 4; ++rt)
+            for (int rt = 0; rt < kTiles; ++rt)
 #pragma unroll
                 for (int ct = 0; ct < W / 16; ++ct) {
                     s4 hv;
@@ -364,17 +379,14 @@ __global__ __launch_bounds__(kNrcBlock) void k_mlp_forward(const float* __restri
                 }
         }
         // output layer
-        const uint16_t* Wo = sW + (NT::resident ? NT::off(L) : 0);
-        if constexpr (!NT::resident) {
-            __syncthreads();
-            stage16(sW, Wt.WT + NT::off(L), NT::k(L) * NT::n(L));
-            __syncthreads();
-        }
+        __syncthreads();
+        stage_rows(sW, Wt.WT + NT::off(L), NT::n(L), NT::k(L));
+        __syncthreads();
         if (!active) continue;
-        f4v acc[4][1];
-        layer_forward<W, kOutCols>(act, LD, Wo, acc, lane);
+        f4v acc[kTiles][1];
+        layer_forward<W, kOutCols>(act, LD, sW, acc, lane);
 #pragma unroll
-        for (int rt = 0; rt < 4; ++rt)
+        for (int rt = 0; rt < kTiles; ++rt)
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 const int r = rt * 16 + q * 4 + j;
@@ -398,7 +410,7 @@ BB_D float loss_grad(float y, float t, float inv_count, float& loss)
 // dz_{l-1} = (dz_l W_l^T) masked by h_l > 0 for a wave's chunk: dz_l
 // (kRows x N) row-major in dzl (LDS), W_l k-major from global memory, h_l
 // (the mask) feature-major from the saved inputs; the result replaces dzl
-// (row-major, stride W) and is stored feature-major to dzc.
+// (row-major, stride ldz) and is stored feature-major to dzc.
 template <class NT, int N>
 BB_D void dz_layer(int l, const uint16_t* hc, const uint16_t* Wk, uint16_t* dzl, uint16_t* dzc, int lane)
 {
@@ -407,14 +419,14 @@ BB_D void dz_layer(int l, const uint16_t* hc, const uint16_t* Wk, uint16_t* dzl,
     const uint16_t* h = hc + NT::act_off(l);
     const uint16_t* Wl = Wk + NT::off(l);
     // the mask first, so that its loads overlap the products
-    s4 hv[4][W / 16];
+    s4 hv[kTiles][W / 16];
 #pragma unroll
-    for (int rt = 0; rt < 4; ++rt)
+    for (int rt = 0; rt < kTiles; ++rt)
 #pragma unroll
         for (int ct = 0; ct < W / 16; ++ct) hv[rt][ct] = load4(h + (ct * 16 + r16) * kRows + rt * 16 + q * 4);
-    f4v acc[4][W / 16];
+    f4v acc[kTiles][W / 16];
 #pragma unroll
-    for (int rt = 0; rt < 4; ++rt)
+    for (int rt = 0; rt < kTiles; ++rt)
 #pragma unroll
         for (int ct = 0; ct < W / 16; ++ct) acc[rt][ct] = f4v{ 0.0f, 0.0f, 0.0f, 0.0f };
     // (rows x N) (N x W): A = dz rows, B = W_l^T (B[n][k] = W_l[k][n])
@@ -424,8 +436,8 @@ BB_D void dz_layer(int l, const uint16_t* hc, const uint16_t* Wk, uint16_t* dzl,
 #pragma unroll
         for (int ct = 0; ct < W / 16; ++ct) b[ct] = load8(Wl + (ct * 16 + r16) * N + kk * 32 + q * 8);
 #pragma unroll
-        for (int rt = 0; rt < 4; ++rt) {
-            const s8v av = load8(dzl + (rt * 16 + r16) * W + kk * 32 + q * 8);
+        for (int rt = 0; rt < kTiles; ++rt) {
+            const s8v av = load8(dzl + (rt * 16 + r16) * NT::ldz + kk * 32 + q * 8);
 #pragma unroll
             for (int ct = 0; ct < W / 16; ++ct) acc[rt][ct] = mfma32(av, b[ct], acc[rt][ct]);
         }
@@ -436,15 +448,15 @@ BB_D void dz_layer(int l, const uint16_t* hc, const uint16_t* Wk, uint16_t* dzl,
 #pragma unroll
         for (int ct = 0; ct < W / 16; ++ct) b[ct] = load4(Wl + (ct * 16 + r16) * N + k0 + q * 4);
 #pragma unroll
-        for (int rt = 0; rt < 4; ++rt) {
-            const s4 av = load4(dzl + (rt * 16 + r16) * W + k0 + q * 4);
+        for (int rt = 0; rt < kTiles; ++rt) {
+            const s4 av = load4(dzl + (rt * 16 + r16) * NT::ldz + k0 + q * 4);
 #pragma unroll
             for (int ct = 0; ct < W / 16; ++ct) acc[rt][ct] = mfma(av, b[ct], acc[rt][ct]);
         }
     }
     uint16_t* out = dzc + NT::dz_off(l - 1);
 #pragma unroll
-    for (int rt = 0; rt < 4; ++rt)
+    for (int rt = 0; rt < kTiles; ++rt)
 #pragma unroll
         for (int ct = 0; ct < W / 16; ++ct) {
             s4 dv;
@@ -454,7 +466,7 @@ BB_D void dz_layer(int l, const uint16_t* hc, const uint16_t* Wk, uint16_t* dzl,
                 const bool on = hj != 0 && !(hj & 0x8000u);
                 const uint16_t d = on ? to_bf16(acc[rt][ct][j]) : uint16_t(0);
                 dv[j] = short(d);
-                dzl[(rt * 16 + q * 4 + j) * W + ct * 16 + r16] = d;
+                dzl[(rt * 16 + q * 4 + j) * NT::ldz + ct * 16 + r16] = d;
             }
             *reinterpret_cast<s4*>(out + (ct * 16 + r16) * kRows + rt * 16 + q * 4) = dv;
         }
@@ -474,7 +486,7 @@ __global__ __launch_bounds__(kNrcBlock) void k_mlp_dz(const float* __restrict__ 
     int off = 0, n = 0;
     span_rows(span, off, n);
     target += size_t(off) * 3;
-    __shared__ __align__(16) uint16_t sD[kNrcBlock / 64][kRows * W]; // dz of the current layer output, row-major
+    __shared__ __align__(16) uint16_t sD[kNrcBlock / 64][kRows * NT::ldz]; // dz of the current layer output, row-major
     __shared__ float sLoss[kNrcBlock / 64];
     static_assert(kNrcBlock / 64 == 4, "four wave sums");
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -489,7 +501,7 @@ __global__ __launch_bounds__(kNrcBlock) void k_mlp_dz(const float* __restrict__ 
         uint16_t* dzc = dzs + size_t(ch) * NT::chunk_dz;
         // dz_L: dL/dy of rows rt*16 + 4q + j, column r16 (3 used)
 #pragma unroll
-        for (int rt = 0; rt < 4; ++rt) {
+        for (int rt = 0; rt < kTiles; ++rt) {
             s4 dv;
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
@@ -499,7 +511,7 @@ __global__ __launch_bounds__(kNrcBlock) void k_mlp_dz(const float* __restrict__ 
                     g = loss_grad(y[size_t(row) * 3 + r16], target[size_t(row) * 3 + r16], inv_count, loss);
                 const uint16_t gb = to_bf16(g);
                 dv[j] = short(gb);
-                dzl[r * W + r16] = gb;
+                dzl[r * NT::ldz + r16] = gb;
             }
             *reinterpret_cast<s4*>(dzc + NT::dz_off(L) + r16 * kRows + rt * 16 + q * 4) = dv;
         }
@@ -528,21 +540,37 @@ BB_D void dw_tile(int l, int mt0, int nt0, int c0, int c1, const uint16_t* acts,
     for (int i = 0; i < TM; ++i)
 #pragma unroll
         for (int j = 0; j < TN; ++j) acc[i][j] = f4v{ 0.0f, 0.0f, 0.0f, 0.0f };
-    for (int c = c0; c < c1; ++c) {
+    constexpr int ST = kRows / 32;
+    s8v a[ST][TM], b[ST][TN];
+    auto fetch = [&](int c) {
         const uint16_t* h = acts + size_t(c) * NT::chunk_acts + NT::act_off(l) + (mt0 * 16 + r16) * kRows + q * 8;
         const uint16_t* d = dzs + size_t(c) * NT::chunk_dz + NT::dz_off(l) + (nt0 * 16 + r16) * kRows + q * 8;
 #pragma unroll
-        for (int st = 0; st < kRows / 32; ++st) {
-            s8v a[TM], b[TN];
+        for (int st = 0; st < ST; ++st) {
 #pragma unroll
-            for (int i = 0; i < TM; ++i) a[i] = load8(h + i * 16 * kRows + st * 32);
+            for (int i = 0; i < TM; ++i) a[st][i] = load8(h + i * 16 * kRows + st * 32);
 #pragma unroll
-            for (int j = 0; j < TN; ++j) b[j] = load8(d + j * 16 * kRows + st * 32);
+            for (int j = 0; j < TN; ++j) b[st][j] = load8(d + j * 16 * kRows + st * 32);
+        }
+    };
+    // the next chunk's operands are on their way while this one's are multiplied
+    if (c0 < c1) fetch(c0);
+    for (int c = c0; c < c1; ++c) {
+        s8v ca[ST][TM], cb[ST][TN];
+#pragma unroll
+        for (int st = 0; st < ST; ++st) {
+#pragma unroll
+            for (int i = 0; i < TM; ++i) ca[st][i] = a[st][i];
+#pragma unroll
+            for (int j = 0; j < TN; ++j) cb[st][j] = b[st][j];
+        }
+        if (c + 1 < c1) fetch(c + 1);
+#pragma unroll
+        for (int st = 0; st < ST; ++st)
 #pragma unroll
             for (int i = 0; i < TM; ++i)
 #pragma unroll
-                for (int j = 0; j < TN; ++j) acc[i][j] = mfma32(a[i], b[j], acc[i][j]);
-        }
+                for (int j = 0; j < TN; ++j) acc[i][j] = mfma32(ca[st][i], cb[st][j], acc[i][j]);
     }
 #pragma unroll
     for (int i = 0; i < TM; ++i)
@@ -553,31 +581,37 @@ BB_D void dw_tile(int l, int mt0, int nt0, int c0, int c1, const uint16_t* acts,
                 out[((mt0 + i) * 16 + q * 4 + e) * N + (nt0 + j) * 16 + r16] = acc[i][j][e];
 }
 
-// dW of every layer as Net::groups work groups times `splits` row ranges,
-// one wave each: block b does group b % groups over chunks
-// [chunks s / splits, chunks (s + 1) / splits) with s = b / groups, into
-// partials[s][params]
+// dW of every layer as Net::groups work groups times `splits` row ranges, one
+// wave each: the waves of block b take unit b % L over chunks
+// [chunks s / splits, chunks (s + 1) / splits) with s = b / L, into
+// partials[s][params].  Unit u < L - 1 is hidden layer u + 1 (its 64 x 64
+// blocks), the last unit layer 0 and the output layer.  Bound by reading the
+// saved activations and gradients, each of which several groups need: the
+// groups of one layer share a block, so that they meet in its CU's cache (56 us
+// with 64-row chunks either way, 39 with 32-row ones, where two waves share a
+// SIMD and the next chunk's operands are fetched while one is multiplied).
 template <class NT>
-__global__ __launch_bounds__(64) void k_mlp_dw(const uint16_t* __restrict__ acts, const uint16_t* __restrict__ dzs,
-                                               RowSpan span, float* __restrict__ partials)
+__global__ __launch_bounds__(64 * NT::dw_waves) void k_mlp_dw(const uint16_t* __restrict__ acts,
+                                                              const uint16_t* __restrict__ dzs, RowSpan span,
+                                                              float* __restrict__ partials)
 {
     constexpr int W = NT::W, L = NT::L, B = W / 64; // 64-wide blocks per hidden dimension
+    static_assert(2 * B <= NT::dw_waves && B * B <= NT::dw_waves, "a unit's groups fit in a block");
     int off = 0, n = 0;
     span_rows(span, off, n);
     const int chunks = (n + kRows - 1) / kRows;
     const int splits = dw_splits(chunks, NT::groups);
-    const int g = blockIdx.x % NT::groups, s = blockIdx.x / NT::groups;
+    const int u = blockIdx.x % L, s = blockIdx.x / L;
     if (n == 0 || s >= splits) return;
     const int c0 = int(int64_t(chunks) * s / splits), c1 = int(int64_t(chunks) * (s + 1) / splits);
-    const int lane = threadIdx.x;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     float* out = partials + size_t(s) * NT::params;
-    if (g < B) { // layer 0: all 80 rows, columns 64 g ..
-        dw_tile<NT, 5, 4>(0, 0, 4 * g, c0, c1, acts, dzs, out + NT::off(0), lane);
-    } else if (g < B + (L - 1) * B * B) {
-        const int i = g - B, l = 1 + i / (B * B), blk = i % (B * B);
-        dw_tile<NT, 4, 4>(l, 4 * (blk / B), 4 * (blk % B), c0, c1, acts, dzs, out + NT::off(l), lane);
-    } else { // output layer: rows 64 (g - ..) .., its 16 columns
-        dw_tile<NT, 4, 1>(L, 4 * (g - B - (L - 1) * B * B), 0, c0, c1, acts, dzs, out + NT::off(L), lane);
+    if (u < L - 1) {
+        if (w < B * B) dw_tile<NT, 4, 4>(1 + u, 4 * (w / B), 4 * (w % B), c0, c1, acts, dzs, out + NT::off(1 + u), lane);
+    } else if (w < B) { // layer 0: all 80 rows, columns 64 w ..
+        dw_tile<NT, 5, 4>(0, 0, 4 * w, c0, c1, acts, dzs, out + NT::off(0), lane);
+    } else if (w < 2 * B) { // output layer: rows 64 (w - B) .., its 16 columns
+        dw_tile<NT, 4, 1>(L, 4 * (w - B), 0, c0, c1, acts, dzs, out + NT::off(L), lane);
     }
 }
 
@@ -1239,7 +1273,7 @@ int train_step(BbNrc* x, const float* inputs_dev, const float* targets_dev, bb::
                            x->y, x->acts);
         hipLaunchKernelGGL(bb::k_mlp_dz<NT>, dim3(grid), dim3(bb::kNrcBlock), 0, st, x->y, targets_dev, span, x->W,
                            x->acts, x->dzs, x->loss_part);
-        hipLaunchKernelGGL(bb::k_mlp_dw<NT>, dim3(NT::groups * bb::dw_splits(chunks, NT::groups)), dim3(64), 0, st,
+        hipLaunchKernelGGL(bb::k_mlp_dw<NT>, dim3(NT::L * bb::dw_splits(chunks, NT::groups)), dim3(64 * NT::dw_waves), 0, st,
                            x->acts, x->dzs, span, x->partials);
         if (!nrc_ok(hipGetLastError(), "k_mlp_dw")) return BBGPU_ERR_DEVICE;
     }
