@@ -167,13 +167,13 @@ def main():
             "kernel": "k_trace_closest (closest-hit traversal of the reference BVH, two levels per fetch)",
             "bound": "hbm",
             # what the counters show (profiles/traversal_c2_counters.md): the
-            # kernel is below the HBM ceiling because of latency and lane
-            # divergence, with measured HBM traffic well under the algorithmic bytes
-            "limiter": "memory latency and lane divergence: 30 of 64 lanes active per VALU instruction, waves "
-                       "waiting 45% of their cycles, L2 hit rate 48%; measured HBM traffic 0.20x the algorithmic "
-                       "bytes (1.89 TB/s), the rest served from L2 and the Infinity Cache, so the algorithmic "
-                       "rate can pass the HBM peak; each launch shares the GPU with the previous depth's shadow "
-                       "traversal (profiles/traversal_c2_counters.md, trace_closest_c2_traffic.md)",
+            # kernel is bound by VALU issue at its lane divergence; its records
+            # are compressed, so it moves far less than the algorithmic bytes
+            "limiter": "VALU issue and lane divergence: 51 and 31 of 64 lanes active per VALU instruction at the "
+                       "first two depths, the VALU busy 76 to 100% of the time; the algorithmic bytes are those of "
+                       "the reference's records, of which the kernel's are a half, mostly served from L1 and L2, so "
+                       "the algorithmic rate can pass the HBM peak; each launch shares the GPU with the previous "
+                       "depth's shadow traversal (profiles/traversal_c2_counters.md)",
             "achieved": round(achieved, 1),
             "peak": HBM_PEAK_GBS,
             "unit": "GB/s",

@@ -531,6 +531,24 @@ bool textures_to_gpu(const BbSceneDesc& d, std::vector<GpuTexture>& out, std::ve
     return true;
 }
 
+// a vector whose elements start uninitialised: every one of them is written
+// afterwards, by the threads of for_each_index, which then take its page faults
+template <typename T>
+struct NoInit : std::allocator<T>
+{
+    template <typename U>
+    struct rebind
+    {
+        using other = NoInit<U>;
+    };
+    template <typename U>
+    void construct(U*) noexcept
+    {
+    }
+};
+template <typename T>
+using RawVector = std::vector<T, NoInit<T>>;
+
 // fn(i) for i in [0, n), on several threads from 2^14 items up; fn(i) writes
 // what belongs to i alone
 template <typename F>
@@ -740,9 +758,9 @@ bool create_scene(const BbSceneDesc& d, BbScene* s, std::string& err)
 
     // BVH slot data
     const int32_t ns = s->n_slots;
-    std::vector<float4> tris(size_t(3) * ns);
-    std::vector<int4> slot_shade(ns);
-    std::vector<int32_t> slot_light(ns);
+    RawVector<float4> tris(size_t(3) * ns);
+    RawVector<int4> slot_shade(ns);
+    RawVector<int32_t> slot_light(ns);
     const std::vector<BbBvhNode>& nodes = bvh.nodes;
     std::atomic<bool> has_null{ false }, alpha_sphere{ false };
     for_each_index(ns, [&](int64_t j) {
@@ -790,7 +808,8 @@ bool create_scene(const BbSceneDesc& d, BbScene* s, std::string& err)
             last.w = i2f(f2i(last.w) | kSlotLast);
         }
     auto ref_of = [&](size_t c) { return nodes[c].count == 0 ? inner_index[c] : ~nodes[c].offset; };
-    std::vector<float4> inner(size_t(4) * std::max(1, n_inner));
+    RawVector<float4> inner(size_t(4) * std::max(1, n_inner));
+    if (n_inner == 0) std::fill(inner.begin(), inner.end(), make_float4(0.0f, 0.0f, 0.0f, 0.0f));
     for_each_index(int64_t(nodes.size()), [&](int64_t i) {
         if (nodes[i].count != 0) return;
         const BbBvhNode& c1 = nodes[i + 1];
@@ -835,7 +854,8 @@ bool create_scene(const BbSceneDesc& d, BbScene* s, std::string& err)
     auto qref_of = [&](size_t c) { return nodes[c].count == 0 ? quad_index[c] : ~nodes[c].offset; };
     // the records, then every leaf's exact box (one upload)
     const size_t quad_vecs = size_t(4) * std::max(1, n_quad);
-    std::vector<uint4> quads(quad_vecs + size_t(2) * ns, make_uint4(0, 0, 0, 0));
+    RawVector<uint4> quads(quad_vecs + size_t(2) * ns);
+    if (n_quad == 0) std::fill(quads.begin(), quads.begin() + long(quad_vecs), make_uint4(0, 0, 0, 0));
     std::atomic<bool> bad_axis{ false };
     for_each_index(n_quad, [&](int64_t qi) {
         const size_t nn = size_t(quad_order[qi]);
@@ -885,15 +905,21 @@ bool create_scene(const BbSceneDesc& d, BbScene* s, std::string& err)
     }
     // the leaves' boxes, and the largest coordinates
     float world_abs[3] = { 0.0f, 0.0f, 0.0f };
-    for (const BbBvhNode& nd : nodes) {
-        if (nd.count == 0) continue;
+    for_each_index(int64_t(nodes.size()), [&](int64_t i) {
+        const BbBvhNode& nd = nodes[i];
+        if (nd.count == 0) return;
         uint4* box = &quads[quad_vecs + 2 * size_t(nd.offset)];
         box[0] = make_uint4(f2u(nd.bmin[0]), f2u(nd.bmin[1]), f2u(nd.bmin[2]), 0);
         box[1] = make_uint4(f2u(nd.bmax[0]), f2u(nd.bmax[1]), f2u(nd.bmax[2]), 0);
+        for (int k = 2; k < 2 * nd.count; ++k) box[k] = make_uint4(0, 0, 0, 0); // (its further slots have none)
+    });
+    // (the root's box holds all others unless some coordinate is not finite)
+    bool finite = true;
+    for (int a = 0; a < 3; ++a) finite = finite && std::isfinite(nodes[0].bmin[a]) && std::isfinite(nodes[0].bmax[a]);
+    for (size_t i = 0; i < (finite ? 1 : nodes.size()); ++i)
         for (int a = 0; a < 3; ++a)
-            for (const float c : { nd.bmin[a], nd.bmax[a] })
+            for (const float c : { nodes[i].bmin[a], nodes[i].bmax[a] })
                 if (std::isfinite(c)) world_abs[a] = std::max(world_abs[a], std::fabs(c));
-    }
 
     // every reference the kernels follow stays inside its array
     auto ref_ok = [&](int32_t ref) { return ref >= 0 ? ref < n_inner : (~ref >= 0 && ~ref < ns); };
@@ -920,7 +946,8 @@ bool create_scene(const BbSceneDesc& d, BbScene* s, std::string& err)
         return false;
     }
 
-    std::vector<float4> normals(std::max(1, d.n_vertices)), tangents(std::max(1, d.n_vertices));
+    RawVector<float4> normals(std::max(1, d.n_vertices)), tangents(std::max(1, d.n_vertices));
+    normals[0] = tangents[0] = make_float4(0.0f, 0.0f, 0.0f, 0.0f); // (a scene without vertices)
     for_each_index(d.n_vertices, [&](int64_t i) {
         normals[i] = make_float4(d.normals[3 * i], d.normals[3 * i + 1], d.normals[3 * i + 2], 0.0f);
         tangents[i] = make_float4(d.tangents[3 * i], d.tangents[3 * i + 1], d.tangents[3 * i + 2], 0.0f);
