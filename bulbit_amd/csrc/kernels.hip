@@ -19,6 +19,7 @@
 // Each path keeps its own PCG32 stream seeded as IndependentSampler does, and
 // draws in the reference's order, so every sample equals the reference's
 // sample up to transcendental rounding.
+#include "bb_index.h"
 #include "bb_shade.h"
 
 #include <algorithm>
@@ -1011,23 +1012,6 @@ struct CacheBufs
     int32_t query_bounce, query_first, query_nee, extra, max_vertices, max_rows, max_queries;
 };
 
-// Pixel number q of the path order: down strips 8 pixels wide, row by row
-// within a strip, so that 64 pixels in a row are an 8 x 8 square.  With the
-// samples of a pixel next to each other too, the rays in flight at one time
-// come from one small part of the image, and so do their first bounces: the
-// traversal kernels read a quarter less from memory, and shading's lanes
-// meet the same material more often (24 of 64 active instead of 21).  The
-// 1080p frame of 64 spp takes 66.3 instead of 68.4 ms, the textured 801 x 451
-// frame of 8 spp 6.6 instead of 7.2, the batch of 8 scenes 64.8 instead of 66.4.
-BB_D void order_pixel(const RenderConsts& rc, int q, int& px, int& py)
-{
-    const int per_strip = 8 * rc.height;
-    const int strip = q / per_strip, r = q - strip * per_strip;
-    const int w = min(8, rc.width - 8 * strip);
-    py = w == 8 ? r >> 3 : r / w;
-    px = 8 * strip + r - py * w;
-}
-
 // UniDirectionalRayIntegrator::Render per (pixel, sample) start
 // (integrator.cpp:187-190): seed, then SampleRay(Next2D(), Next2D()) with the
 // lens sample u1 drawn first (argument evaluation of the reference's compiler),
@@ -1043,7 +1027,7 @@ __global__ __launch_bounds__(kShadeBlock) void k_raygen(GpuCamera cam, RenderCon
     int px, py, sample = *rc.sample_begin + rc.sample0;
     if (rc.pass_spp > 0) {
         const int q = i / rc.pass_spp;
-        order_pixel(rc, q, px, py);
+        order_pixel(rc.width, rc.height, q, px, py);
         sample += i - q * rc.pass_spp;
     } else {
         const int pix = i % rc.npix;
@@ -1689,7 +1673,7 @@ __global__ __launch_bounds__(kShadeBlock) void k_film(RenderConsts rc, const flo
     int p = q;
     if (rc.pass_spp > 0 && on) {
         int px, py;
-        order_pixel(rc, q, px, py);
+        order_pixel(rc.width, rc.height, q, px, py);
         p = py * rc.width + px;
     }
     float sr = 0.0f, sg = 0.0f, sb = 0.0f;
