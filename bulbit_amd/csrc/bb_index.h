@@ -3,6 +3,8 @@
 // (kernels.hip) and a host-side test (compiled with g++).
 #pragma once
 
+#include <stddef.h>
+
 #if defined(__HIPCC__)
 #define BB_INDEX __host__ __device__ inline
 #else
@@ -32,5 +34,18 @@ BB_INDEX void order_pixel(int width, int height, int q, int& px, int& py)
     py = w == 8 ? r >> 3 : r / w;
     px = 8 * strip + r - py * w;
 }
+
+// where ray i of a batch starts in an array of 16-byte vectors, two to a ray
+BB_INDEX size_t ray_at(int i) { return 2 * size_t(i); }
+
+// where pixel p starts in a film's sums, three floats to a pixel
+BB_INDEX size_t film_at(int p) { return 3 * size_t(p); }
+
+// the query that an idle lane takes from its wave's claimed ones, [rb, re), as
+// the rank-th of the idle lanes (0 to 63); -1 when there are not that many
+BB_INDEX int claim(int rb, int re, int rank) { return rank < re - rb ? rb + rank : -1; }
+
+// the first claimed query left over once n_idle lanes (up to 64) have taken theirs
+BB_INDEX int claims_left(int rb, int re, int n_idle) { return n_idle < re - rb ? rb + n_idle : re; }
 
 } // namespace bb

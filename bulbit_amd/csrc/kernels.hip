@@ -712,13 +712,14 @@ BB_D void persistent_trace(const SceneView& S, const Src& src, int n, int* fetch
                 if (n_idle == 64 && !more) break;
                 if (n_idle == 64) continue;
             }
-            const int mine = rb + __popcll(idle & below);
-            if (L.cur == kNoRef && mine < re) {
-                id = mine;
-                src.load(id, L);
-                lane_root<COUNT>(S, L, c);
+            if (L.cur == kNoRef) {
+                id = claim(rb, re, __popcll(idle & below));
+                if (id >= 0) {
+                    src.load(id, L);
+                    lane_root<COUNT>(S, L, c);
+                }
             }
-            rb = min(rb + n_idle, re);
+            rb = claims_left(rb, re, n_idle);
         }
         for (;;) {
             if (L.cur >= 0) {
@@ -827,7 +828,8 @@ struct BatchSrc
     int any_hit;
     BB_D void load(int i, Lane& L) const
     {
-        const float4 r0 = rays[2 * i], r1 = rays[2 * i + 1];
+        const float4* r = rays + ray_at(i);
+        const float4 r0 = r[0], r1 = r[1];
         lane_start(L, xyz(r0), xyz(r1), r0.w, r1.w);
     }
     BB_D void finish(int i, const Lane& L) const
@@ -1679,9 +1681,10 @@ __global__ __launch_bounds__(kShadeBlock) void k_film(RenderConsts rc, const flo
     float sr = 0.0f, sg = 0.0f, sb = 0.0f;
     int32_t cnt = 0;
     if (on) {
-        sr = film_sum[3 * p];
-        sg = film_sum[3 * p + 1];
-        sb = film_sum[3 * p + 2];
+        const float* f = film_sum + film_at(p);
+        sr = f[0];
+        sg = f[1];
+        sb = f[2];
         cnt = film_count[p];
     }
     auto add = [&](float4 l) {
@@ -1712,9 +1715,10 @@ __global__ __launch_bounds__(kShadeBlock) void k_film(RenderConsts rc, const flo
         for (int pid = q; pid < rc.n_paths; pid += rc.npix) add(L[pid]);
     }
     if (!on) return;
-    film_sum[3 * p] = sr;
-    film_sum[3 * p + 1] = sg;
-    film_sum[3 * p + 2] = sb;
+    float* f = film_sum + film_at(p);
+    f[0] = sr;
+    f[1] = sg;
+    f[2] = sb;
     film_count[p] = cnt;
 }
 

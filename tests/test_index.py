@@ -48,3 +48,18 @@ def test_path_order_of_the_largest_images(probe, width, height):
     n = width * height
     qs = sorted({q for k in range(33) for q in (n * k // 32 - 1, n * k // 32, n * k // 32 + 1) if 0 <= q < n})
     assert probe("pixel", [(width, height, q) for q in qs]) == [_pixel(width, height, q) for q in qs]
+
+
+# a batch takes up to 2^31 - 1 rays of two vectors each, an image 2^30 pixels of three floats
+def test_places_of_the_last_rays_and_pixels(probe):
+    rays = [0, 1, 2 ** 30 - 1, 2 ** 30, 2 ** 31 - 1]
+    assert probe("ray", [(i,) for i in rays]) == [(2 * i,) for i in rays]
+    pixels = [0, 1, 2 ** 31 // 3, 2 ** 31 // 3 + 1, 2 ** 30 - 1]
+    assert probe("film", [(p,) for p in pixels]) == [(3 * p,) for p in pixels]
+
+
+def test_claims_up_to_the_last_query(probe):
+    most = 2 ** 31 - 1
+    cases = [(rb, re, n) for end in (128, most) for re in (end - 64, end - 1, end) for rb in range(re - 66, re + 1)
+             for n in (0, 1, 31, 63, 64)]
+    assert probe("claim", cases) == [(rb + n if rb + n < re else -1, min(rb + n, re)) for rb, re, n in cases]
