@@ -175,8 +175,9 @@ struct SceneView
     // no node counters: record of internal node N holds the entries of N's
     // children, an inner child replaced by its own two children (so up to 4
     // entries: node N's grandchildren, or a child that is a leaf).  Their
-    // boxes are rounded outwards to 8 bits per plane on a grid of the record,
-    // planes at p + q 2^e on each axis, packed one byte per entry:
+    // boxes, relative to the scene's centre, are rounded outwards to 8 bits per
+    // plane on a grid of the record (bb_slab.h), planes at p + q 2^e on each
+    // axis, packed one byte per entry:
     //   {p.x, p.y, p.z, e.x | e.y << 8 | e.z << 16 (signed bytes)}
     //   {min.x, min.y, min.z, order}  {max.x, max.y, max.z, 0}
     //   {ref0, ref1, ref2, ref3}
@@ -188,7 +189,11 @@ struct SceneView
     // comes before entry 0 (child1's), entry 3 before entry 2 (child2's).
     const uint4* quads;
     const float4* leaf_box; // 2 per slot, at a leaf's first slot: its exact box {min, 0} {max, 0}
-    float world_abs[3];     // largest finite coordinate of any box, per axis
+    // What a ray starts with, in memory rather than among the kernels'
+    // arguments, which are kept in scalar registers throughout: {the scene's
+    // centre, far_away} {half, 0} (slab_ray: every box lies within centre +-
+    // half), the root's box {min, 0} {max, 0}
+    const float4* root;
     int32_t quad_root;        // the root as a two-level reference (record 0, or a leaf)
     int32_t quad_stack_depth; // most stack entries a two-level traversal holds (+ 1)
 };

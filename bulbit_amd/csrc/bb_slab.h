@@ -1,0 +1,276 @@
+// bb_slab.h — box tests of the traversal: RayCast's own, and those of the
+// two-level records, whose boxes are rounded outwards and tested with a margin;
+// shared by the kernels (kernels.hip), the scene set-up (host.cpp) and a
+// host-side test (compiled with g++).  V is a vector of three floats x, y, z.
+//
+// The records are compressed wide nodes in the manner of Ylitie, Karras and
+// Laine, "Efficient Incoherent Ray Traversal on GPUs Through Compressed Wide
+// BVHs" (HPG 2017): an origin and a power of two per axis, a byte per plane.
+#pragma once
+
+#include <float.h>
+#include <math.h>
+#include <stdint.h>
+#include <string.h>
+
+#if defined(__HIPCC__)
+#define BB_SLAB __host__ __device__ __forceinline__
+#else
+#define BB_SLAB inline
+#endif
+
+namespace bb
+{
+
+// ------------------------------------------------------------ the exact test
+
+// AABB3::TestRay with precomputed inverse direction (bounding_box.h:443-484),
+// split into the part that does not depend on t_max and the box's entry
+// distance.
+//
+// The reference tests x, then y against the x-tightened interval, then z
+// against the x,y-tightened interval, and ignores any NaN slab distance
+// (every comparison with NaN is false).  Unrolled, it fails exactly when one
+// of these pairs is out of order:
+//   t_min  > t_max_i  (i = x, y, z)      t_min_i > t_max          (i = x, y, z)
+//   t_min_i > t_max_j (i != j)
+// (t_min is never compared with t_max, and t_min_i <= t_max_i always holds
+// for one axis because both are computed with the same sign of inv.)  With
+// NaN-ignoring max/min over the three axes, lo = max_i t_min_i and
+// hi = min_i t_max_i, that is
+//   fail = t_min > hi  or  lo > hi  or  lo > t_max.
+// The first two do not involve t_max.  The last is monotone in t_max: a box
+// that fails it fails again for any smaller t_max, and whether it passes
+// later needs only lo, which does not change.
+struct BoxHit
+{
+    bool ok;  // the t_max-independent part passed
+    float lo; // entry distance: the box passes iff ok and !(lo > t_max)
+};
+
+template <class V>
+BB_SLAB BoxHit box_part(V bmin, V bmax, V o, float t_min, V inv, bool n0, bool n1, bool n2)
+{
+    const float lx = ((n0 ? bmax.x : bmin.x) - o.x) * inv.x;
+    const float hx = ((n0 ? bmin.x : bmax.x) - o.x) * inv.x;
+    const float ly = ((n1 ? bmax.y : bmin.y) - o.y) * inv.y;
+    const float hy = ((n1 ? bmin.y : bmax.y) - o.y) * inv.y;
+    const float lz = ((n2 ? bmax.z : bmin.z) - o.z) * inv.z;
+    const float hz = ((n2 ? bmin.z : bmax.z) - o.z) * inv.z;
+    BoxHit h;
+    h.lo = fmaxf(fmaxf(lx, ly), lz);
+    const float hi = fminf(fminf(hx, hy), hz);
+    h.ok = !((t_min > hi) | (h.lo > hi));
+    return h;
+}
+
+BB_SLAB bool box_pass(BoxHit h, float t_max) { return h.ok && !(h.lo > t_max); }
+
+// ------------------------------------------------------- tests with a margin
+
+// The constants of a ray for box tests that need no division.  Planes are taken
+// relative to the scene's centre c; with o' = o - c the slab distance of one at
+// B' = B - c is
+//   near = fma(B', inv, near0),  near0 = -o' inv - M
+//   far  = fma(B', inv, far0),   far0  = -o' inv + M
+// per axis, so that a box test passes whenever the exact one of a box inside
+// does.
+// half: every box lies within c +- half; rcp: 1 / d to one unit in the last
+// place.
+//
+// With S = |o'| + half on an axis and u = 2^-24 the errors are, in units of
+// u S |inv|: o' one, the reciprocal two, near0 one, the two fused operations (a
+// record's plane is one more, quad_entry) one each, the exact test's reciprocal,
+// subtraction and product one each; M is over 13.  It grows with the distance
+// from the scene, not with the coordinates: a batch of 1 M rays on 328 K
+// triangles takes 260 us wherever the scene lies (with planes as they are and
+// M from |o|: 260 us around the origin, 1,540 moved by 10^4 times its size on
+// each axis, 22,600 by 10^5).
+//
+// An axis the direction hardly moves along has an inverse so large that the
+// distances overflow or, at the origin's own plane, are not a number; there
+// |inv| is cut to 2^40 times the smallest of the three.  With t the distance at
+// which the ray has left the scene, M is 4 t more on such an axis: a slab that
+// holds the origin spans more than [-t, t] and decides nothing, as in the exact
+// test, and one that the origin lies outside of by more than M's share still
+// fails.
+//
+// False where this does not hold: for rays that
+// are not finite, and for those whose distances or inverses come near the ends
+// of the type's range.  Such a ray is tested exactly, on one-level records.  So
+// is one that starts further than `far_away` from the scene (the sum over the
+// axes), where M, 8e-7 of that distance, would pass too many boxes.
+template <class V>
+BB_SLAB bool slab_ray(V o, V rcp, V centre, V half, float far_away, V& inv, V& near0, V& far0)
+{
+    const float ox = o.x - centre.x, oy = o.y - centre.y, oz = o.z - centre.z;
+    const float ax = fabsf(rcp.x), ay = fabsf(rcp.y), az = fabsf(rcp.z);
+    const float sx = fabsf(ox) + half.x, sy = fabsf(oy) + half.y, sz = fabsf(oz) + half.z;
+    const float least = fminf(fminf(ax, ay), az), most = least * 0x1p40f;
+    const float s = sx + sy + sz, t = s * least;
+    const float tiny = fmaf(most, 0x1p-125f, 1e-36f); // a grid's smallest step, and what underflows
+    const float add = fmaf(4.0f, t, tiny);
+    const bool cx = ax > most, cy = ay > most, cz = az > most;
+    const float bx = cx ? most : ax, by = cy ? most : ay, bz = cz ? most : az;
+    inv.x = copysignf(bx, rcp.x);
+    inv.y = copysignf(by, rcp.y);
+    inv.z = copysignf(bz, rcp.z);
+    const float mx = fmaf(sx * bx, 8e-7f, cx ? add : tiny);
+    const float my = fmaf(sy * by, 8e-7f, cy ? add : tiny);
+    const float mz = fmaf(sz * bz, 8e-7f, cz ? add : tiny);
+    near0.x = fmaf(-ox, inv.x, -mx);
+    near0.y = fmaf(-oy, inv.y, -my);
+    near0.z = fmaf(-oz, inv.z, -mz);
+    far0.x = fmaf(-ox, inv.x, mx);
+    far0.y = fmaf(-oy, inv.y, my);
+    far0.z = fmaf(-oz, inv.z, mz);
+    return (s < far_away) & (t < 1e20f) & (least > 1e-30f) & (least < 1e25f);
+}
+
+// The test of the scene's own box with the margin
+template <class V>
+BB_SLAB bool slab_root(V half, V inv, V near0, V far0, float t_min, float t_max)
+{
+    const float lo = fmaxf(fmaxf(fmaf(-half.x, fabsf(inv.x), near0.x), fmaf(-half.y, fabsf(inv.y), near0.y)),
+                           fmaf(-half.z, fabsf(inv.z), near0.z));
+    const float hi = fminf(fminf(fmaf(half.x, fabsf(inv.x), far0.x), fmaf(half.y, fabsf(inv.y), far0.y)),
+                           fmaf(half.z, fabsf(inv.z), far0.z));
+    return !((t_min > hi) | (lo > hi) | (lo > t_max));
+}
+
+// ---------------------------------------------------------- two-level records
+
+// v 2^e
+BB_SLAB float slab_scale(float v, int e)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __builtin_amdgcn_ldexpf(v, e);
+#else
+    return ldexpf(v, e);
+#endif
+}
+
+// What the four entries of a record (SceneView::quads) share for one ray: the
+// near and far distance of the grid's origin, the distance between its planes, and the packed rows of the planes that the ray meets first and last
+template <class V>
+struct QuadSlabs
+{
+    V n, f, s;
+    uint32_t nx, ny, nz, fx, fy, fz;
+};
+
+// p: the grid's origin, e: its exponents, min and max: the entries' planes
+template <class V>
+BB_SLAB QuadSlabs<V> quad_slabs(V p, uint32_t e, uint32_t min_x, uint32_t min_y, uint32_t min_z, uint32_t max_x,
+                                uint32_t max_y, uint32_t max_z, V inv, V near0, V far0, bool n0, bool n1, bool n2)
+{
+    QuadSlabs<V> q;
+    q.n.x = fmaf(p.x, inv.x, near0.x);
+    q.n.y = fmaf(p.y, inv.y, near0.y);
+    q.n.z = fmaf(p.z, inv.z, near0.z);
+    q.f.x = fmaf(p.x, inv.x, far0.x);
+    q.f.y = fmaf(p.y, inv.y, far0.y);
+    q.f.z = fmaf(p.z, inv.z, far0.z);
+    q.s.x = slab_scale(inv.x, int8_t(e));
+    q.s.y = slab_scale(inv.y, int8_t(e >> 8));
+    q.s.z = slab_scale(inv.z, int8_t(e >> 16));
+    q.nx = n0 ? max_x : min_x;
+    q.fx = n0 ? min_x : max_x;
+    q.ny = n1 ? max_y : min_y;
+    q.fy = n1 ? min_y : max_y;
+    q.nz = n2 ? max_z : min_z;
+    q.fz = n2 ? min_z : max_z;
+    return q;
+}
+
+// byte E of a packed row as a float
+template <int E>
+BB_SLAB float quad_byte(uint32_t row)
+{
+    return float((row >> (8 * E)) & 0xffu);
+}
+
+// entry E: false when the exact test of every box inside its own fails, else
+// lo is at most the entry distance of each of them
+template <int E, class V>
+BB_SLAB bool quad_entry(const QuadSlabs<V>& q, float t_min, float t_max, float& lo)
+{
+    lo = fmaxf(fmaxf(fmaf(quad_byte<E>(q.nx), q.s.x, q.n.x), fmaf(quad_byte<E>(q.ny), q.s.y, q.n.y)),
+               fmaf(quad_byte<E>(q.nz), q.s.z, q.n.z));
+    const float hi = fminf(fminf(fmaf(quad_byte<E>(q.fx), q.s.x, q.f.x), fmaf(quad_byte<E>(q.fy), q.s.y, q.f.y)),
+                           fmaf(quad_byte<E>(q.fz), q.s.z, q.f.z));
+    return !((t_min > hi) | (lo > hi) | (lo > t_max));
+}
+
+// One axis of a record: the grid p + q 2^e, relative to the scene's centre, and
+// the entries' planes rounded outwards to it, a byte per entry (a missing entry
+// gets an empty range)
+struct QuadGrid
+{
+    float p;
+    int8_t e;
+    uint32_t lo, hi;
+};
+
+// bmin, bmax: the entries' boxes on the axis; has: which entries there are
+inline QuadGrid quad_grid(const float bmin[4], const float bmax[4], const bool has[4], float centre)
+{
+    QuadGrid g{ 0.0f, 0, 0, 0 };
+    double lo = HUGE_VAL, hi = -HUGE_VAL;
+    bool finite = true;
+    for (int k = 0; k < 4; ++k) {
+        if (!has[k]) continue;
+        finite = finite && fabsf(bmin[k]) <= FLT_MAX && fabsf(bmax[k]) <= FLT_MAX;
+        if (bmin[k] < lo) lo = bmin[k];
+        if (bmax[k] > hi) hi = bmax[k];
+    }
+    if (!finite) { // planes beyond every ray: the axis never fails a box
+        g.p = -FLT_MAX;
+        g.e = 127;
+        for (int k = 0; k < 4; ++k)
+            if (has[k]) g.hi |= 255u << (8 * k);
+        return g;
+    }
+    // the lowest plane, rounded down
+    lo -= centre;
+    hi -= centre;
+    g.p = float(lo);
+    if (double(g.p) > lo) g.p = nextafterf(g.p, -INFINITY);
+    lo = g.p;
+    // 2^e > (hi - lo) / 255, from the exponent bits
+    const double step = (hi - lo) / 255.0;
+    uint64_t bits;
+    memcpy(&bits, &step, 8);
+    int e = step > 0.0 ? int(bits >> 52) - 1022 : 0;
+    if (e < -126) e = -126;
+    if (e > 127) e = 127;
+    bits = uint64_t(1023 - e) << 52; // 2^-e
+    double inv;
+    memcpy(&inv, &bits, 8);
+    for (int k = 0; k < 4; ++k) {
+        uint32_t a = 255, b = 0;
+        if (has[k]) {
+            const double x = (double(bmin[k]) - centre - lo) * inv, y = (double(bmax[k]) - centre - lo) * inv;
+            a = uint32_t(x);
+            if (a > 255u) a = 255u;
+            b = uint32_t(y);
+            if (double(b) < y) b += 1u;
+            if (b > 255u) b = 255u;
+        }
+        g.lo |= a << (8 * k);
+        g.hi |= b << (8 * k);
+    }
+    g.e = int8_t(e);
+    return g;
+}
+
+// The largest distance from `centre` of a plane of [bmin, bmax], rounded up
+inline float slab_half(float bmin, float bmax, float centre)
+{
+    const double a = double(centre) - bmin, b = double(bmax) - centre;
+    const double d = a > b ? a : b;
+    const float f = float(d);
+    return double(f) < d ? nextafterf(f, INFINITY) : f;
+}
+
+} // namespace bb

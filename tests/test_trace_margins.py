@@ -1,0 +1,125 @@
+"""Rays at the ends of the float range, and from far away, on triangles, spheres
+and alpha-tested triangles: the traversal without node counters (two-level
+records, or one-level ones where those cannot serve) against the oracle, bit
+for bit where the hit's distance is a number."""
+import os
+
+import numpy as np
+import pytest
+
+from bulbit_amd import scenes
+from test_textures import textured_scene
+
+THREADS = max(1, min(16, len(os.sched_getaffinity(0))))
+
+
+def _spheres():
+    """64 spheres in a box, so that there are records above the leaves"""
+    sc, _ = scenes.readme_scene(64, 36)
+    rng = np.random.default_rng(9)
+    for _ in range(63):
+        sc.add_sphere(tuple(float(x) for x in rng.uniform(-2, 2, 3)), float(rng.uniform(0.05, 0.5)), 0)
+    return sc
+
+
+@pytest.fixture(scope="module")
+def pairs():
+    from bulbit_amd.gpu import GpuScene
+    from oracle import OracleScene
+
+    made = {}
+
+    def get(name):
+        if name not in made:
+            sc = {"triangles": lambda: scenes.icosphere_scene(level=3)[0], "spheres": _spheres,
+                  "alpha": lambda: textured_scene(level=4)[0]}[name]()
+            made[name] = GpuScene(sc), OracleScene(sc)
+        return made[name]
+
+    return get
+
+
+KINDS = ["plain", "axis", "long", "tiny", "zero", "far", "very_far", "infinite", "nan"]
+
+
+def _rays(kind, lo, hi, n=30_000):
+    seed = KINDS.index(kind)
+    rng = np.random.default_rng(300 + seed)
+    rays = scenes.random_rays(lo, hi, n, seed=400 + seed)
+    i, axis = np.arange(n), rng.integers(0, 3, n)
+    size = float(np.linalg.norm(np.asarray(hi) - np.asarray(lo)))
+    if kind == "axis":
+        d = 10.0 ** rng.uniform(-44, -5, (n, 3)) * np.where(rng.random((n, 3)) < 0.5, 1, -1)
+        d[i, axis] = np.where(rng.random(n) < 0.5, 1.0, -1.0)
+        rays["d"] = d.astype(np.float32)
+    elif kind in ("long", "tiny"):
+        a, b = (0, 37) if kind == "long" else (-44, -10)
+        length = 10.0 ** rng.uniform(a, b, n)
+        rays["d"] = (rays["d"] * length[:, None]).astype(np.float32)
+        rays["t_min"] = 0.0
+        some = rng.random(n) < 0.3
+        with np.errstate(over="ignore"):
+            rays["t_max"][some] = (size * rng.uniform(0, 2, n) / length)[some].astype(np.float32)
+    elif kind == "zero":
+        rays["d"] = np.where(rng.random((n, 3)) < 0.5, 0.0, -0.0).astype(np.float32)
+        rays["t_max"] = np.where(rng.random(n) < 0.5, np.inf, 1.0)
+    elif kind in ("far", "very_far"):
+        away = size * 10.0 ** (rng.uniform(1, 6, n) if kind == "far" else rng.uniform(6, 36, n))
+        if kind == "very_far":  # along an axis, so that something is hit
+            rays["d"] = 0.0
+            rays["d"][i, axis] = np.where(rng.random(n) < 0.5, 1.0, -1.0)
+        rays["o"] = (rays["o"] - rays["d"] * away[:, None]).astype(np.float32)
+    elif kind == "infinite":
+        rays["o"][i, axis] = np.where(rng.random(n) < 0.5, np.inf, -np.inf)
+        rays["d"][i, rng.integers(0, 3, n)] = np.inf
+    elif kind == "nan":
+        rays["o"][i[::2], axis[::2]] = np.nan
+        rays["d"][i[1::2], axis[1::2]] = np.nan
+    return rays
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("scene", ["triangles", "spheres", "alpha"])
+@pytest.mark.parametrize("kind", KINDS)
+def test_rays_at_the_ends_of_the_range(pairs, scene, kind):
+    if scene == "alpha" and kind in ("zero", "very_far", "infinite", "nan"):
+        pytest.skip("the reference's texture lookup at coordinates that are not numbers is undefined")
+    g, o = pairs(scene)
+    rays = _rays(kind, *o.world_bounds())
+    for any_hit in (False, True):
+        print(scene, kind, any_hit, flush=True)
+        hits, _ = g.trace(rays, any_hit=any_hit)
+        want, _ = o.trace(rays, any_hit=any_hit, threads=THREADS)
+        if any_hit:
+            assert np.array_equal(hits["prim"], want["prim"])
+        else:
+            # A hit at a distance that is not a number (overflow in the shape's
+            # test) bounds nothing: which primitive keeps it is not compared
+            number = ~np.isnan(want["t"])
+            assert np.array_equal(hits["prim"] >= 0, want["prim"] >= 0)
+            assert np.array_equal(~np.isnan(hits["t"]), number)
+            for f in ("prim", "t", "u", "v"):
+                assert np.array_equal(hits[f].view(np.int32)[number], want[f].view(np.int32)[number]), f
+        if kind in ("plain", "axis", "long", "far", "very_far"):
+            assert np.any(want["prim"] >= 0)
+
+
+# the same scene anywhere: box tests relative to its centre
+@pytest.mark.gpu
+@pytest.mark.parametrize("move", [(0.0, 0.0, 0.0), (1e3, -2e4, 5.0), (-1e5, 1e5, 1e5)])
+@pytest.mark.parametrize("any_hit", [False, True])
+def test_scene_away_from_the_origin(move, any_hit):
+    from bulbit_amd.gpu import GpuScene
+    from oracle import OracleScene
+
+    sc, _ = scenes.icosphere_scene(level=4)
+    sc.positions = (sc.positions.astype(np.float64) + move).astype(np.float32)
+    g, o = GpuScene(sc), OracleScene(sc)
+    rays = scenes.random_rays(*o.world_bounds(), 50_000, seed=11, t_max=3.0 if any_hit else np.inf)
+    hits, _ = g.trace(rays, any_hit=any_hit)
+    want, _ = o.trace(rays, any_hit=any_hit, threads=THREADS)
+    assert np.mean(want["prim"] >= 0) > 0.01
+    assert np.array_equal(hits["prim"], want["prim"])
+    if not any_hit:
+        for f in ("t", "u", "v"):
+            assert np.array_equal(hits[f].view(np.int32), want[f].view(np.int32)), f
