@@ -212,6 +212,8 @@ struct QuadGrid
     uint32_t lo, hi;
 };
 
+inline double clamp_byte(double x) { return x < 0.0 ? 0.0 : (x > 255.0 ? 255.0 : x); }
+
 // bmin, bmax: the entries' boxes on the axis; has: which entries there are
 inline QuadGrid quad_grid(const float bmin[4], const float bmax[4], const bool has[4], float centre)
 {
@@ -224,13 +226,7 @@ inline QuadGrid quad_grid(const float bmin[4], const float bmax[4], const bool h
         if (bmin[k] < lo) lo = bmin[k];
         if (bmax[k] > hi) hi = bmax[k];
     }
-    if (!finite) { // planes beyond every ray: the axis never fails a box
-        g.p = -FLT_MAX;
-        g.e = 127;
-        for (int k = 0; k < 4; ++k)
-            if (has[k]) g.hi |= 255u << (8 * k);
-        return g;
-    }
+    if (!finite) return g; // the scene's box is not finite then: no ray walks its records (slab_ray)
     // the lowest plane, rounded down
     lo -= centre;
     hi -= centre;
@@ -250,12 +246,12 @@ inline QuadGrid quad_grid(const float bmin[4], const float bmax[4], const bool h
     for (int k = 0; k < 4; ++k) {
         uint32_t a = 255, b = 0;
         if (has[k]) {
-            const double x = (double(bmin[k]) - centre - lo) * inv, y = (double(bmax[k]) - centre - lo) * inv;
+            // (outside [0, 255] only for a box that is inverted, which no ray meets)
+            const double x = clamp_byte((double(bmin[k]) - centre - lo) * inv);
+            const double y = clamp_byte((double(bmax[k]) - centre - lo) * inv);
             a = uint32_t(x);
-            if (a > 255u) a = 255u;
             b = uint32_t(y);
             if (double(b) < y) b += 1u;
-            if (b > 255u) b = 255u;
         }
         g.lo |= a << (8 * k);
         g.hi |= b << (8 * k);

@@ -410,7 +410,8 @@ BB_D QEnt qsel(bool c, QEnt a, QEnt b) { return QEnt{ c ? a.ref : b.ref, c ? a.l
 // with the same t_max.  A leaf RayCast would not have visited can change
 // nothing unless one of its primitives is accepted, and before a primitive
 // is accepted the leaf's exact box is tested (leaf_visited): a leaf's box
-// lies inside its ancestors', whose slab intervals are then no smaller (the
+// lies inside its ancestors' (bounds hold no NaN: they grow from an empty box
+// by comparisons that drop it), whose slab intervals are then no smaller (the
 // float slab distances are monotone in the plane coordinates, NaN counting
 // as ignored), so that one test decides whether RayCast reaches the leaf.
 // Hits are RayCast's bit for bit; only the node-test count differs, so the

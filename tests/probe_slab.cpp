@@ -44,8 +44,24 @@ static bool entry(const bb::QuadSlabs<V>& q, float t_min, float t_max, float& lo
     return bb::quad_entry<E>(q, t_min, t_max, lo);
 }
 
+// One axis of a record from eight numbers, the entries' planes (bmin bmax), and
+// the centre: prints the grid and the packed rows
+static int grid(char** argv)
+{
+    float lo[4], hi[4];
+    for (int k = 0; k < 4; ++k) {
+        lo[k] = std::strtof(argv[2 + 2 * k], nullptr);
+        hi[k] = std::strtof(argv[3 + 2 * k], nullptr);
+    }
+    const bool has[4] = { true, true, true, true };
+    const bb::QuadGrid q = bb::quad_grid(lo, hi, has, std::strtof(argv[10], nullptr));
+    std::printf("%.9g %d %u %u\n", q.p, q.e, q.lo, q.hi);
+    return 0;
+}
+
 int main(int argc, char** argv)
 {
+    if (argc == 11) return grid(argv);
     const char* scene = argv[1];
     const char* kind = argv[2];
     g.seed(std::strtoul(argv[3], nullptr, 10));

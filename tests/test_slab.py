@@ -15,13 +15,13 @@ RAYS = ["plain", "axis", "far", "length", "any"]
 @pytest.fixture(scope="module")
 def probe(tmp_path_factory):
     exe = str(tmp_path_factory.mktemp("slab") / "probe_slab")
-    subprocess.run(["g++", "-std=c++17", "-O2", "-ffp-contract=off", "-fsanitize=undefined",
+    subprocess.run(["g++", "-std=c++17", "-O2", "-ffp-contract=off", "-fsanitize=undefined,float-cast-overflow",
                     "-fno-sanitize-recover=all", "-o", exe, os.path.join(HERE, "probe_slab.cpp")], check=True)
 
-    def run(scene, rays, seed):
-        out = subprocess.run([exe, scene, rays, str(seed)], capture_output=True, text=True)
+    def run(*args):
+        out = subprocess.run([exe] + [str(a) for a in args], capture_output=True, text=True)
         assert out.returncode == 0, out.stderr
-        return [int(x) for x in out.stdout.split()]
+        return [float(x) if args[0] == "grid" else int(x) for x in out.stdout.split()]
 
     return run
 
@@ -46,3 +46,18 @@ def test_no_box_is_lost(probe, scene, rays):
 def test_margins_are_narrow(probe, scene, rays):
     tests, _, _, _, loose = probe(scene, rays, 7)
     assert loose < 0.01 * tests
+
+
+# boxes that are accepted but hold nothing: inverted ones (spheres of negative radius) beside ordinary ones and
+# alone, and ones that are not finite; the grid's conversions stay in range, and ordinary entries keep their planes
+@pytest.mark.parametrize("odd", [(5.0, -5.0), (1e30, -1e30), (0.5, 0.25), ("nan", 1.0), (0.0, "inf"), ("-inf", "nan")])
+@pytest.mark.parametrize("all_odd", [False, True])
+def test_grid_of_odd_boxes(probe, odd, all_odd):
+    boxes = [odd] * 4 if all_odd else [(-1.0, 0.0), odd, (0.25, 2.0), odd]
+    p, e, lo, hi = probe("grid", *[x for b in boxes for x in b], 0.5)
+    if all_odd or "nan" in odd or "inf" in odd:
+        return
+    for k in (0, 2):
+        low, high = (p + ((int(row) >> (8 * k)) & 255) * 2.0 ** e + 0.5 for row in (lo, hi))
+        step = 2.0 ** e
+        assert boxes[k][0] - step <= low <= boxes[k][0] and boxes[k][1] <= high <= boxes[k][1] + step

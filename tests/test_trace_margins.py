@@ -123,3 +123,56 @@ def test_scene_away_from_the_origin(move, any_hit):
     if not any_hit:
         for f in ("t", "u", "v"):
             assert np.array_equal(hits[f].view(np.int32), want[f].view(np.int32)), f
+
+
+def _row(odd):
+    """triangles in a row along x, some with a coordinate that is not a number;
+    or spheres, some of negative radius"""
+    sc, _ = scenes.readme_scene(64, 36)
+    if odd == "negative radius":
+        rng = np.random.default_rng(21)
+        for i in range(48):
+            r = float(rng.uniform(0.05, 0.4))
+            sc.add_sphere((0.5 * i - 12.0, 1.0, float(rng.uniform(-0.2, 0.2))), -r if i % 3 == 0 else r, 0)
+        return sc
+    x = np.arange(64) * 0.5 - 16.0
+    p = np.zeros((64, 3, 3), np.float32)
+    p[:, :, 0] = x[:, None] + np.array([0.0, 0.4, 0.2])
+    p[:, :, 1] = np.array([0.5, 0.5, 1.5])
+    p[:, 2, 2] = 0.1
+    p[5::16, 0, 1] = np.nan  # (in the first vertex: the bounds of the triangle drop it in the others)
+    n = np.tile(np.float32([0, 0, 1]), (192, 1))
+    t = np.tile(np.float32([1, 0, 0]), (192, 1))
+    sc.add_mesh(p.reshape(-1, 3), n, t, np.arange(192, dtype=np.int32).reshape(-1, 3), np.zeros(64, np.int32))
+    return sc
+
+
+# Shapes whose box is inverted (a coordinate that is not a number leaves the
+# bounds as they start, empty): nothing meets them, and the boxes beside them in
+# a record keep their planes.  Rays at and just outside the row's upper edge
+@pytest.mark.gpu
+@pytest.mark.parametrize("odd", ["nan", "negative radius"])
+@pytest.mark.parametrize("any_hit", [False, True])
+def test_shapes_without_proper_boxes(odd, any_hit):
+    from bulbit_amd.gpu import GpuScene
+    from oracle import OracleScene
+
+    sc = _row(odd)
+    g, o = GpuScene(sc), OracleScene(sc)
+    rng = np.random.default_rng(31)
+    n = 40_000
+    rays = scenes.random_rays((-16, 0, -4), (16, 2, 4), n, seed=32)
+    rays["o"][::2, 1] = 1.5 + rng.uniform(-0.02, 0.02, n // 2)
+    rays["d"][::2] = np.float32([0.02, 0.001, -1.0]) * np.where(rng.random(n // 2) < 0.5, 1, -1)[:, None]
+    rays["t_min"] = 0.0
+    if any_hit:
+        rays["t_max"] = 3.0
+    hits, _ = g.trace(rays, any_hit=any_hit)
+    want, _ = o.trace(rays, any_hit=any_hit, threads=THREADS)
+    assert 0.01 < np.mean(want["prim"] >= 0) < 0.99
+    assert np.array_equal(hits["prim"] >= 0, want["prim"] >= 0)
+    if not any_hit:
+        number = ~np.isnan(want["t"])
+        assert np.array_equal(~np.isnan(hits["t"]), number)
+        for f in ("prim", "t", "u", "v"):
+            assert np.array_equal(hits[f].view(np.int32)[number], want[f].view(np.int32)[number]), f
