@@ -549,12 +549,13 @@ struct NoInit : std::allocator<T>
 template <typename T>
 using RawVector = std::vector<T, NoInit<T>>;
 
-// fn(i) for i in [0, n), on several threads from 2^14 items up; fn(i) writes
-// what belongs to i alone
+// fn(i) for i in [0, n), on several threads from 2^16 items up (a scene of
+// 20,500 triangles is set up in 4.78 ms, with threads from 2^14 items in 5.25);
+// fn(i) writes what belongs to i alone
 template <typename F>
 void for_each_index(int64_t n, F fn)
 {
-    const int64_t threads = std::min<int64_t>({ n >> 13, 8, int64_t(std::max(1u, std::thread::hardware_concurrency())) });
+    const int64_t threads = std::min<int64_t>({ n >> 15, 8, int64_t(std::max(1u, std::thread::hardware_concurrency())) });
     auto part = [&](int64_t k, int64_t of) {
         for (int64_t i = n * k / of; i < n * (k + 1) / of; ++i) fn(i);
     };
@@ -758,8 +759,23 @@ bool create_scene(const BbSceneDesc& d, BbScene* s, std::string& err)
     auto ref_of = [&](size_t c) { return nodes[c].count == 0 ? inner_index[c] : ~nodes[c].offset; };
     RawVector<float4> inner(size_t(4) * std::max(1, n_inner));
     if (n_inner == 0) std::fill(inner.begin(), inner.end(), make_float4(0.0f, 0.0f, 0.0f, 0.0f));
+    // SceneView::root, every leaf's exact box and the two-level records, one
+    // upload: the boxes are written with the one-level records, whose pass
+    // takes the same turns (room for as many two-level ones as there can be)
+    const size_t quad_vecs = (4 + size_t(2) * ns + 3) / 4 * 4; // the records start on a cache line
+    RawVector<uint4> walk(quad_vecs + size_t(4) * std::max(1, n_inner));
+    walk[quad_vecs - 2] = walk[quad_vecs - 1] = make_uint4(0, 0, 0, 0); // (what may lie between)
+    uint4* const leaf_box = walk.data() + 4;
+    uint4* const quads = walk.data() + quad_vecs;
     for_each_index(int64_t(nodes.size()), [&](int64_t i) {
-        if (nodes[i].count != 0) return;
+        const BbBvhNode& nd = nodes[i];
+        if (nd.count != 0) {
+            uint4* box = leaf_box + 2 * size_t(nd.offset);
+            box[0] = make_uint4(f2u(nd.bmin[0]), f2u(nd.bmin[1]), f2u(nd.bmin[2]), 0);
+            box[1] = make_uint4(f2u(nd.bmax[0]), f2u(nd.bmax[1]), f2u(nd.bmax[2]), 0);
+            for (int k = 2; k < 2 * nd.count; ++k) box[k] = make_uint4(0, 0, 0, 0); // (its further slots have none)
+            return;
+        }
         const BbBvhNode& c1 = nodes[i + 1];
         const BbBvhNode& c2 = nodes[size_t(nodes[i].offset)];
         float4* r = &inner[size_t(4) * inner_index[i]];
@@ -800,15 +816,13 @@ bool create_scene(const BbSceneDesc& d, BbScene* s, std::string& err)
     }
     const int32_t n_quad = int32_t(quad_order.size());
     auto qref_of = [&](size_t c) { return nodes[c].count == 0 ? quad_index[c] : ~nodes[c].offset; };
-    // the records, then every leaf's exact box, then SceneView::root (one upload)
-    const size_t quad_vecs = size_t(4) * std::max(1, n_quad);
-    RawVector<uint4> quads(quad_vecs + size_t(2) * ns + 4);
-    if (n_quad == 0) std::fill(quads.begin(), quads.begin() + long(quad_vecs), make_uint4(0, 0, 0, 0));
+    if (n_quad == 0) std::fill(quads, quads + 4, make_uint4(0, 0, 0, 0));
     float centre[3], half[3];
     for (int a = 0; a < 3; ++a) {
         centre[a] = float(0.5 * (double(nodes[0].bmin[a]) + double(nodes[0].bmax[a])));
         half[a] = slab_half(nodes[0].bmin[a], nodes[0].bmax[a], centre[a]);
     }
+    static_assert(offsetof(BbBvhNode, bmax) == 12 && sizeof(BbBvhNode) >= 28, "quad_grid reads seven floats of a node");
     std::atomic<bool> bad_axis{ false };
     for_each_index(n_quad, [&](int64_t qi) {
         const size_t nn = size_t(quad_order[qi]);
@@ -835,49 +849,33 @@ bool create_scene(const BbSceneDesc& d, BbScene* s, std::string& err)
         }
         int32_t ref[4];
         for (int e = 0; e < 4; ++e) ref[e] = has[e] ? qref_of(ent[e]) : INT32_MIN;
-        QuadGrid g[3];
-        for (int a = 0; a < 3; ++a) {
-            float bmin[4], bmax[4];
-            for (int e = 0; e < 4; ++e) {
-                bmin[e] = nodes[ent[e]].bmin[a];
-                bmax[e] = nodes[ent[e]].bmax[a];
-            }
-            g[a] = quad_grid(bmin, bmax, has, centre[a]);
-        }
+        const float* box[4];
+        for (int e = 0; e < 4; ++e) box[e] = nodes[ent[has[e] ? e : e - 1]].bmin; // (bmax follows)
+        const QuadGrid g = quad_grid(box, has, centre);
         // bit 3 o for every octant o that is negative along the axis
         constexpr uint32_t kNegative[3] = { 0x208208u, 0x240240u, 0x249000u };
         const uint32_t order = kNegative[axes[0]] | (inner_child[0] ? kNegative[axes[1]] << 1 : 0u) |
                                (inner_child[1] ? kNegative[axes[2]] << 2 : 0u);
         uint4* r = &quads[size_t(4) * qi];
-        r[0] = make_uint4(f2u(g[0].p), f2u(g[1].p), f2u(g[2].p),
-                          uint32_t(uint8_t(g[0].e)) | uint32_t(uint8_t(g[1].e)) << 8 | uint32_t(uint8_t(g[2].e)) << 16);
-        r[1] = make_uint4(g[0].lo, g[1].lo, g[2].lo, order);
-        r[2] = make_uint4(g[0].hi, g[1].hi, g[2].hi, 0);
+        r[0] = make_uint4(f2u(g.p[0]), f2u(g.p[1]), f2u(g.p[2]),
+                          uint32_t(uint8_t(g.e[0])) | uint32_t(uint8_t(g.e[1])) << 8 | uint32_t(uint8_t(g.e[2])) << 16);
+        r[1] = make_uint4(g.lo[0], g.lo[1], g.lo[2], order);
+        r[2] = make_uint4(g.hi[0], g.hi[1], g.hi[2], 0);
         r[3] = make_uint4(uint32_t(ref[0]), uint32_t(ref[1]), uint32_t(ref[2]), uint32_t(ref[3]));
     });
     if (bad_axis) {
         err = "internal error: BVH split axis out of range";
         return false;
     }
-    // the leaves' boxes
-    for_each_index(int64_t(nodes.size()), [&](int64_t i) {
-        const BbBvhNode& nd = nodes[i];
-        if (nd.count == 0) return;
-        uint4* box = &quads[quad_vecs + 2 * size_t(nd.offset)];
-        box[0] = make_uint4(f2u(nd.bmin[0]), f2u(nd.bmin[1]), f2u(nd.bmin[2]), 0);
-        box[1] = make_uint4(f2u(nd.bmax[0]), f2u(nd.bmax[1]), f2u(nd.bmax[2]), 0);
-        for (int k = 2; k < 2 * nd.count; ++k) box[k] = make_uint4(0, 0, 0, 0); // (its further slots have none)
-    });
-
-    // Rays from where the margins of their box tests (slab_ray: 8e-7 of the
+    // Rays from where the margins of their box tests (slab_ray: 9e-7 of the
     // distance) come to about a third of a leaf's size meet too many boxes.
     // Batches of 1 M rays, two-level against one-level walk: leaves 0.01 wide,
     // from 3,000 away 376 and 456 us, from 10,000 692 and 497; 0.08 wide, from
     // 10,000 away 209 and 291, from 100,000 300 and 291.  The size is the
-    // geometric mean over up to 512 leaves (width + height + depth).
+    // geometric mean over up to 128 leaves (width + height + depth).
     double log_size = 0.0;
     int sampled = 0;
-    for (size_t i = 0; i < nodes.size(); i += 1 + nodes.size() / 512) {
+    for (size_t i = 0; i < nodes.size(); i += 1 + nodes.size() / 128) {
         size_t j = i;
         while (nodes[j].count == 0) ++j; // (child1 comes next: down to a leaf)
         double size = 1e-30;
@@ -886,7 +884,7 @@ bool create_scene(const BbSceneDesc& d, BbScene* s, std::string& err)
         ++sampled;
     }
     const float far_away = float(std::min(4e5 * std::exp2(log_size / sampled), 1e30));
-    uint4* root = &quads[quad_vecs + 2 * size_t(ns)];
+    uint4* const root = walk.data();
     root[0] = make_uint4(f2u(centre[0]), f2u(centre[1]), f2u(centre[2]), f2u(far_away));
     root[1] = make_uint4(f2u(half[0]), f2u(half[1]), f2u(half[2]), 0);
     root[2] = make_uint4(f2u(nodes[0].bmin[0]), f2u(nodes[0].bmin[1]), f2u(nodes[0].bmin[2]), 0);
@@ -932,13 +930,15 @@ bool create_scene(const BbSceneDesc& d, BbScene* s, std::string& err)
         V.root_box[3 + k] = nodes[0].bmax[k];
     }
     V.root_ref = ref_of(0);
-    if (!upload(s, quads.data(), quads.size(), &V.quads, err)) return false;
+    const uint4* walk_dev = nullptr;
+    if (!upload(s, walk.data(), quad_vecs + size_t(4) * std::max(1, n_quad), &walk_dev, err)) return false;
+    V.root = reinterpret_cast<const float4*>(walk_dev);
+    V.leaf_box = V.root + 4;
+    V.quads = walk_dev + quad_vecs;
     V.quad_root = qref_of(0);
     // each record leaves at most 3 entries on the stack beside the one taken
     // next, which is pushed too
     V.quad_stack_depth = 3 * quad_levels + 1;
-    V.leaf_box = reinterpret_cast<const float4*>(V.quads + quad_vecs);
-    V.root = V.leaf_box + 2 * size_t(ns);
     if (!upload(s, tris.data(), tris.size(), &V.tris, err)) return false;
     if (!upload(s, slot_shade.data(), slot_shade.size(), &V.slot_shade, err)) return false;
     if (!upload(s, slot_light.data(), slot_light.size(), &V.slot_light, err)) return false;

@@ -44,18 +44,21 @@ static bool entry(const bb::QuadSlabs<V>& q, float t_min, float t_max, float& lo
     return bb::quad_entry<E>(q, t_min, t_max, lo);
 }
 
-// One axis of a record from eight numbers, the entries' planes (bmin bmax), and
-// the centre: prints the grid and the packed rows
+// A record's grid on one axis from eight numbers, the entries' planes (bmin
+// bmax), and the centre: prints the grid and the packed rows
 static int grid(char** argv)
 {
-    float lo[4], hi[4];
+    float box[4][7] = {};
+    const float* at[4];
     for (int k = 0; k < 4; ++k) {
-        lo[k] = std::strtof(argv[2 + 2 * k], nullptr);
-        hi[k] = std::strtof(argv[3 + 2 * k], nullptr);
+        box[k][0] = std::strtof(argv[2 + 2 * k], nullptr);
+        box[k][3] = std::strtof(argv[3 + 2 * k], nullptr);
+        at[k] = box[k];
     }
     const bool has[4] = { true, true, true, true };
-    const bb::QuadGrid q = bb::quad_grid(lo, hi, has, std::strtof(argv[10], nullptr));
-    std::printf("%.9g %d %u %u\n", q.p, q.e, q.lo, q.hi);
+    const float centre[3] = { std::strtof(argv[10], nullptr), 0.0f, 0.0f };
+    const bb::QuadGrid q = bb::quad_grid(at, has, centre);
+    std::printf("%.9g %d %u %u\n", q.p[0], q.e[0], q.lo[0], q.hi[0]);
     return 0;
 }
 
@@ -143,15 +146,22 @@ int main(int argc, char** argv)
         const bool n0 = ri.x < 0.0f, n1 = ri.y < 0.0f, n2 = ri.z < 0.0f;
         for (int b = 0; b < 64; b += 4) {
             const bool has[4] = { true, b % 8 == 0, true, true };
-            bb::QuadGrid q[3];
-            for (int a = 0; a < 3; ++a) {
-                const float lo[4] = { mn[b][a], mn[b + 1][a], mn[b + 2][a], mn[b + 3][a] };
-                const float hi[4] = { mx[b][a], mx[b + 1][a], mx[b + 2][a], mx[b + 3][a] };
-                q[a] = bb::quad_grid(lo, hi, has, centre[a]);
+            float box[4][7];
+            const float* at[4];
+            for (int k = 0; k < 4; ++k) {
+                const int from = has[k] ? b + k : b; // (a missing entry repeats another)
+                for (int a = 0; a < 3; ++a) {
+                    box[k][a] = mn[from][a];
+                    box[k][3 + a] = mx[from][a];
+                }
+                box[k][6] = NAN;
+                at[k] = box[k];
             }
-            const uint32_t e = uint32_t(uint8_t(q[0].e)) | uint32_t(uint8_t(q[1].e)) << 8 | uint32_t(uint8_t(q[2].e)) << 16;
-            const bb::QuadSlabs<V> s = bb::quad_slabs(V{ q[0].p, q[1].p, q[2].p }, e, q[0].lo, q[1].lo, q[2].lo, q[0].hi,
-                                                      q[1].hi, q[2].hi, inv, near0, far0, n0, n1, n2);
+            const float at_centre[3] = { centre.x, centre.y, centre.z };
+            const bb::QuadGrid q = bb::quad_grid(at, has, at_centre);
+            const uint32_t e = uint32_t(uint8_t(q.e[0])) | uint32_t(uint8_t(q.e[1])) << 8 | uint32_t(uint8_t(q.e[2])) << 16;
+            const bb::QuadSlabs<V> s = bb::quad_slabs(V{ q.p[0], q.p[1], q.p[2] }, e, q.lo[0], q.lo[1], q.lo[2], q.hi[0],
+                                                      q.hi[1], q.hi[2], inv, near0, far0, n0, n1, n2);
             for (int k = 0; k < 4; ++k) {
                 if (!has[k]) continue;
                 const bb::BoxHit h = bb::box_part(mn[b + k], mx[b + k], o, t_min, ei, e0, e1, e2);
