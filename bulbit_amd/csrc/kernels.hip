@@ -62,9 +62,13 @@ constexpr int kLeafMin = 16;
 constexpr int kLeafShare = 2;
 // waves per SIMD the traversal kernels are built for (72 VGPRs): left to
 // itself the compiler took 87 and five waves fitted (72.6 ms per 1080p frame
-// of 64 spp; six 70.1, seven 68.8, eight, with spills, 70.8).  Not the
-// kernels with the alpha test, which spill (textured 801 x 451 frame of 8
-// spp: 6.6 ms without the bound, 7.1 at six, 7.6 at seven).
+// of 64 spp; six 70.1, seven 68.8, eight, with spills, 70.8).  Shadow rays run
+// at seven; closest hits at 26 waves per CU, six and a half, since the LDS of
+// their stacks (12,288 bytes a block) fits 13 times.  Not the kernels with the
+// alpha test, which would spill: they run at four or five as they come
+// (textured 801 x 451 frame of 8 spp, when first measured: 6.6 ms without the
+// bound, 7.1 at six, 7.6 at seven; bound to five now 5.62 instead of 5.58, and
+// a batch of 1 M closest hits 278 us instead of 260).
 constexpr int kTraceWaves = 7;
 constexpr int kLdsCdfEntries = 2049; // lights whose CDF the shading kernel keeps in LDS (up to 2048)
 constexpr int kMaxGridBlocks = 256 * 32;
@@ -1167,17 +1171,21 @@ BB_D void cache_features(const CacheBufs& C, const GpuMaterial& m, f3 p, f3 wo, 
 constexpr int kKindsLcd = (1 << MK_LAMBERT) | (1 << MK_CONDUCTOR) | (1 << MK_DIELECTRIC);
 constexpr int kKindsMr = (1 << MK_METALLIC_ROUGHNESS) | (1 << MK_LAMBERT);
 
-// Waves per SIMD that shading with every BxDF is built for: left alone the
-// compiler takes 297 VGPRs for the textured kernel and one wave fits (801 x
-// 451 frame of 8 spp, textures in every slot: 6.5 ms; bound to three, with
-// some spills, 5.7; to four 6.0).  The kernels for fewer kinds need 154 and
-// 155 and are best left alone (Lambertian + conductor + dielectric bound to
-// four: the 1080p frame of 64 spp 67.4 instead of 65.8 ms).
-constexpr int kShadeWavesAll = 3;
+// Waves per SIMD that shading with every BxDF is built for, with some spills:
+// left alone the compiler takes 256 VGPRs and more, and one wave fits.  One /
+// two / three waves, all spp and 8 bounces: 801 x 451 with textures in every
+// slot, 8 spp, 6.5 ms alone, 5.7 at three, 6.0 at four; without textures 4.65 /
+// 3.98 / 3.94 ms; cached frames, which keep more of a path's state, with
+// textures 4.29 / 3.74 / 3.97 ms at 1601 x 901 x 4 spp (64-wide network) and
+// 3.02 / 2.80 / 2.91 at 801 x 451 x 2 (128-wide), without them 3.65 / 3.21 /
+// 3.24.  The kernels for fewer kinds need 146 to 156 and are best left alone
+// (Lambertian + conductor + dielectric bound to four: the 1080p frame of 64 spp
+// 67.4 instead of 65.8 ms).
+constexpr int kShadeWavesAll = 3, kShadeWavesAllCached = 2;
 
 // KM: the BxDF kinds compiled in (the scene's materials' kinds, or all)
 template <bool CACHE, bool TEX, int KM>
-__global__ __launch_bounds__(kShadeBlock, KM == kAllKinds ? kShadeWavesAll : 1) void k_shade(SceneView S, RenderConsts rc, PathBufs P, int depth, CacheBufs C)
+__global__ __launch_bounds__(kShadeBlock, KM == kAllKinds ? (CACHE ? kShadeWavesAllCached : kShadeWavesAll) : 1) void k_shade(SceneView S, RenderConsts rc, PathBufs P, int depth, CacheBufs C)
 {
     const int in = depth & 1, out = in ^ 1;
     const int n = P.counts[4 * depth];
