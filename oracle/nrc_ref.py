@@ -84,16 +84,17 @@ def forward(w, raw):
     return y, hs
 
 
-def loss_and_grad(w, raw, target):
-    """relative L2 loss and its gradient with respect to the flat weights"""
+def loss_and_grad(w, raw, target, rows=None):
+    """relative L2 loss and its gradient with respect to the flat weights, as a
+    mean over `rows` rows (those given unless the batch has more)"""
     y, hs = forward(w, raw)
     W = [bf16(m) for m in split(np.asarray(w, np.float32))]
     hidden = len(W) - 1
-    n = len(raw)
+    n = len(raw) if rows is None else rows
     d = y - target
     den = y * y + 0.01
     loss = float(np.sum(d * d / den) / (3 * n))
-    dz = np.zeros((n, OUT_COLS), np.float32)
+    dz = np.zeros((len(raw), OUT_COLS), np.float32)
     dz[:, :3] = bf16((2.0 * d / den / (3 * n)).astype(np.float32))
     grads = [None] * (hidden + 1)
     for l in range(hidden, -1, -1):
