@@ -73,14 +73,12 @@ struct Net
     static constexpr int n(int l) { return l == L ? kOutCols : W; }
     static constexpr int off(int l) { return l == 0 ? 0 : off(l - 1) + k(l - 1) * n(l - 1); }
     static constexpr int params = off(L + 1);
-    // row strides (bf16) of the tiles in LDS of the training step's forward
-    // pass (a wave's activations, a layer's staged weights) and gradient chain:
-    // eight more than the row, since rows of 256 bytes start in one bank and
-    // the operand reads, 16 rows at a time, met 16 deep (forward kernel over
-    // 65,536 rows 53 -> 45 us)
-    static constexpr int ld = (W > kIn ? W : kIn) + kPad;
-    static constexpr int ldz = W + kPad;
-    static constexpr int max_layer = W * (W > kIn ? W + kPad : kIn + kPad);
+    // row stride (bf16) of the tiles in LDS of the wide network's training step,
+    // in the forward pass (a wave's activations, a layer's staged weights) and
+    // the gradient chain: eight more than the row, since rows of 256 bytes
+    // start in one bank and the operand reads, 16 rows at a time, met 16 deep
+    // (forward kernel over 65,536 rows 53 -> 45 us)
+    static constexpr int ld = W + kPad;
     // Layer inputs saved by the training forward pass, per chunk of kRows
     // rows, feature-major ([feature][row in chunk]): h_0 (kIn features), then
     // h_1..h_L (W each).  Eight consecutive rows of one feature are one 16-byte
@@ -95,7 +93,7 @@ struct Net
     // 80 x 64 blocks (5 x 4 tiles), the hidden layers in 64 x 64 blocks,
     // the output layer in 64 x 16 blocks
     static constexpr int groups = W / 64 + (L - 1) * (W / 64) * (W / 64) + W / 64;
-    static constexpr int dw_waves = W / 64 > 1 ? (W / 64) * (W / 64) : 2; // waves of a dW block
+    static constexpr int dw_waves = (W / 64) * (W / 64); // waves of a dW block
     // The query kernel's weights: per layer, W_l^T cut into the A-operand
     // fragments of v_mfma_f32_16x16x32_bf16 (16 output features x 32 input
     // features, K padded to a multiple of 32), fragment (l, k-step, m-tile)
@@ -310,11 +308,11 @@ struct NrcWeights
     const uint16_t* W;  // bf16 [k][n] per layer
 };
 
-// y = f(enc(raw)) for n rows; with SAVE the bf16 input of every layer is
-// stored per chunk, feature-major (Net::act_off), for the backward pass.
-// The block's four waves take four consecutive chunks per iteration; when
-// the weights are staged layer by layer every wave joins every barrier.
-template <class NT, bool SAVE>
+// y = f(enc(raw)) for n rows; the bf16 input of every layer is stored per
+// chunk, feature-major (Net::act_off), for the backward pass.  The block's four
+// waves take four consecutive chunks per iteration; the weights are staged
+// layer by layer, and every wave joins every barrier.
+template <class NT>
 __global__ __launch_bounds__(kNrcBlock) void k_mlp_forward(const float* __restrict__ raw, RowSpan span, NrcWeights Wt,
                                                             float* __restrict__ out, uint16_t* __restrict__ acts)
 {
@@ -322,9 +320,10 @@ __global__ __launch_bounds__(kNrcBlock) void k_mlp_forward(const float* __restri
     int off = 0, n = 0;
     span_rows(span, off, n);
     raw += size_t(off) * kRawStride;
-    __shared__ __align__(16) uint16_t sW[NT::max_layer];
+    __shared__ __align__(16) uint16_t sW[W * LD]; // a layer's weights
     __shared__ __align__(16) uint16_t sAct[kNrcBlock / 64][kRows * LD];
     static_assert(kIn % 8 == 0 && W % 8 == 0, "weights staged 16 bytes at a time");
+    static_assert(kIn <= W, "the first layer's rows are no longer than the others'");
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     uint16_t* act = sAct[wave];
     const int r16 = lane & 15, q = lane >> 4;
@@ -342,9 +341,8 @@ __global__ __launch_bounds__(kNrcBlock) void k_mlp_forward(const float* __restri
                     encode_row(raw + size_t(row) * kRawStride, e);
                 else
                     for (int i = 0; i < kIn; ++i) e[i] = 0;
-                if (SAVE) // every row of the chunk, zeros beyond n
-                    for (int i = 0; i < kIn; ++i)
-                        acts[size_t(ch) * NT::chunk_acts + NT::act_off(0) + i * kRows + lane] = e[i];
+                for (int i = 0; i < kIn; ++i) // every row of the chunk, zeros beyond n
+                    acts[size_t(ch) * NT::chunk_acts + NT::act_off(0) + i * kRows + lane] = e[i];
             }
         }
         // hidden layers in a rolled loop (one copy of the code: small kernels
@@ -373,9 +371,8 @@ __global__ __launch_bounds__(kNrcBlock) void k_mlp_forward(const float* __restri
                         hv[j] = short(h);
                     }
                     // rows rt*16 + 4q .. +3 of feature ct*16 + r16 of h_{l+1}
-                    if (SAVE)
-                        *reinterpret_cast<s4*>(acts + size_t(ch) * NT::chunk_acts + NT::act_off(l + 1) +
-                                               (ct * 16 + r16) * kRows + rt * 16 + q * 4) = hv;
+                    *reinterpret_cast<s4*>(acts + size_t(ch) * NT::chunk_acts + NT::act_off(l + 1) +
+                                           (ct * 16 + r16) * kRows + rt * 16 + q * 4) = hv;
                 }
         }
         // output layer
@@ -410,7 +407,7 @@ BB_D float loss_grad(float y, float t, float inv_count, float& loss)
 // dz_{l-1} = (dz_l W_l^T) masked by h_l > 0 for a wave's chunk: dz_l
 // (kRows x N) row-major in dzl (LDS), W_l k-major from global memory, h_l
 // (the mask) feature-major from the saved inputs; the result replaces dzl
-// (row-major, stride ldz) and is stored feature-major to dzc.
+// (row-major, stride ld) and is stored feature-major to dzc.
 template <class NT, int N>
 BB_D void dz_layer(int l, const uint16_t* hc, const uint16_t* Wk, uint16_t* dzl, uint16_t* dzc, int lane)
 {
@@ -437,7 +434,7 @@ BB_D void dz_layer(int l, const uint16_t* hc, const uint16_t* Wk, uint16_t* dzl,
         for (int ct = 0; ct < W / 16; ++ct) b[ct] = load8(Wl + (ct * 16 + r16) * N + kk * 32 + q * 8);
 #pragma unroll
         for (int rt = 0; rt < kTiles; ++rt) {
-            const s8v av = load8(dzl + (rt * 16 + r16) * NT::ldz + kk * 32 + q * 8);
+            const s8v av = load8(dzl + (rt * 16 + r16) * NT::ld + kk * 32 + q * 8);
 #pragma unroll
             for (int ct = 0; ct < W / 16; ++ct) acc[rt][ct] = mfma32(av, b[ct], acc[rt][ct]);
         }
@@ -449,7 +446,7 @@ BB_D void dz_layer(int l, const uint16_t* hc, const uint16_t* Wk, uint16_t* dzl,
         for (int ct = 0; ct < W / 16; ++ct) b[ct] = load4(Wl + (ct * 16 + r16) * N + k0 + q * 4);
 #pragma unroll
         for (int rt = 0; rt < kTiles; ++rt) {
-            const s4 av = load4(dzl + (rt * 16 + r16) * NT::ldz + k0 + q * 4);
+            const s4 av = load4(dzl + (rt * 16 + r16) * NT::ld + k0 + q * 4);
 #pragma unroll
             for (int ct = 0; ct < W / 16; ++ct) acc[rt][ct] = mfma(av, b[ct], acc[rt][ct]);
         }
@@ -466,7 +463,7 @@ BB_D void dz_layer(int l, const uint16_t* hc, const uint16_t* Wk, uint16_t* dzl,
                 const bool on = hj != 0 && !(hj & 0x8000u);
                 const uint16_t d = on ? to_bf16(acc[rt][ct][j]) : uint16_t(0);
                 dv[j] = short(d);
-                dzl[(rt * 16 + q * 4 + j) * NT::ldz + ct * 16 + r16] = d;
+                dzl[(rt * 16 + q * 4 + j) * NT::ld + ct * 16 + r16] = d;
             }
             *reinterpret_cast<s4*>(out + (ct * 16 + r16) * kRows + rt * 16 + q * 4) = dv;
         }
@@ -486,7 +483,7 @@ __global__ __launch_bounds__(kNrcBlock) void k_mlp_dz(const float* __restrict__ 
     int off = 0, n = 0;
     span_rows(span, off, n);
     target += size_t(off) * 3;
-    __shared__ __align__(16) uint16_t sD[kNrcBlock / 64][kRows * NT::ldz]; // dz of the current layer output, row-major
+    __shared__ __align__(16) uint16_t sD[kNrcBlock / 64][kRows * NT::ld]; // dz of the current layer output, row-major
     __shared__ float sLoss[kNrcBlock / 64];
     static_assert(kNrcBlock / 64 == 4, "four wave sums");
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -511,7 +508,7 @@ __global__ __launch_bounds__(kNrcBlock) void k_mlp_dz(const float* __restrict__ 
                     g = loss_grad(y[size_t(row) * 3 + r16], target[size_t(row) * 3 + r16], inv_count, loss);
                 const uint16_t gb = to_bf16(g);
                 dv[j] = short(gb);
-                dzl[r * NT::ldz + r16] = gb;
+                dzl[r * NT::ld + r16] = gb;
             }
             *reinterpret_cast<s4*>(dzc + NT::dz_off(L) + r16 * kRows + rt * 16 + q * 4) = dv;
         }
@@ -1269,7 +1266,7 @@ int train_step(BbNrc* x, const float* inputs_dev, const float* targets_dev, bb::
         const bb::NrcWeights Wt{ x->WT, x->W };
         const int grid = nrc_grid(max_len);
         nloss = grid;
-        hipLaunchKernelGGL((bb::k_mlp_forward<NT, true>), dim3(grid), dim3(bb::kNrcBlock), 0, st, inputs_dev, span, Wt,
+        hipLaunchKernelGGL(bb::k_mlp_forward<NT>, dim3(grid), dim3(bb::kNrcBlock), 0, st, inputs_dev, span, Wt,
                            x->y, x->acts);
         hipLaunchKernelGGL(bb::k_mlp_dz<NT>, dim3(grid), dim3(bb::kNrcBlock), 0, st, x->y, targets_dev, span, x->W,
                            x->acts, x->dzs, x->loss_part);
