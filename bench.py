@@ -166,14 +166,16 @@ def main():
         "roofline": {
             "kernel": "k_trace_closest (closest-hit traversal of the reference BVH, two levels per fetch)",
             "bound": "hbm",
-            # what the counters show (profiles/traversal_c2_counters.md): the
-            # kernel is bound by VALU issue at its lane divergence; its records
-            # are compressed, so it moves far less than the algorithmic bytes
-            "limiter": "VALU issue and lane divergence: 51 and 31 of 64 lanes active per VALU instruction at the "
-                       "first two depths, the VALU busy 76 to 100% of the time; the algorithmic bytes are those of "
-                       "the reference's records, of which the kernel's are a half, mostly served from L1 and L2, so "
-                       "the algorithmic rate can pass the HBM peak; each launch shares the GPU with the previous "
-                       "depth's shadow traversal (profiles/traversal_c2_counters.md)",
+            # what the counters show (profiles/traversal_c2_counters.md): lanes
+            # diverge while the vector units hardly have a free turn; its
+            # records are compressed, so it moves far less than the
+            # algorithmic bytes
+            "limiter": "lane divergence at a high instruction rate: 51 and 32 of 64 lanes active per VALU instruction "
+                       "at the first two depths, 0.19 and 0.27 VALU instructions per SIMD and cycle (0.25 is one "
+                       "every four cycles), half of a wave's cycles waiting; the algorithmic bytes are those of the "
+                       "reference's records, of which the kernel's are a half, mostly served from L1 and L2, so the "
+                       "algorithmic rate can pass the HBM peak; each launch shares the GPU with the previous depth's "
+                       "shadow traversal (profiles/traversal_c2_counters.md)",
             "achieved": round(achieved, 1),
             "peak": HBM_PEAK_GBS,
             "unit": "GB/s",

@@ -176,8 +176,8 @@ struct SceneView
     // children, an inner child replaced by its own two children (so up to 4
     // entries: node N's grandchildren, or a child that is a leaf).  Their
     // boxes, relative to the scene's centre, are rounded outwards to 8 bits per
-    // plane on a grid of the record (bb_slab.h), planes at p + q 2^e on each
-    // axis, packed one byte per entry:
+    // plane on a grid of the record, as in published compressed wide BVHs (named
+    // in bb_slab.h), planes at p + q 2^e on each axis, packed one byte per entry:
     //   {p.x, p.y, p.z, e.x | e.y << 8 | e.z << 16 (signed bytes)}
     //   {min.x, min.y, min.z, order}  {max.x, max.y, max.z, 0}
     //   {ref0, ref1, ref2, ref3}

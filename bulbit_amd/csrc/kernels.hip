@@ -2,14 +2,16 @@
 // launch them: batch traversal (bbgpu_trace) and the wavefront path tracer
 // (bbgpu_render).
 //
-// Traversal follows BVH::RayCast (include/bulbit/bvh.h:101-155) exactly: LIFO
-// stack seeded with the root, box test when a node is taken with the current
-// t_max, leaf primitives in stored order, far child pushed and near child
-// taken next (near = child2 when the ray direction along the split axis is
-// negative).  Taking the near child directly instead of pushing and popping it
-// tests the same nodes in the same order with the same t_max.  The stack lives
-// in LDS, laid out [depth][thread] so that the 64 lanes of a wave touch 64
-// consecutive words.
+// Traversal visits the leaves that BVH::RayCast (include/bulbit/bvh.h:101-155)
+// visits, in its order and with its t_max, and tests their primitives in stored
+// order, so hits are its own bit for bit.  Kernels with node counters walk the
+// BVH's own nodes as RayCast does: the far child pushed, the near one (child2
+// when the ray direction along the split axis is negative) taken next.  The
+// others walk two-level records with compressed boxes (quad_expand): the entries
+// that pass are pushed in reverse order and the next one is popped; RayCast's
+// box test of a leaf is made before one of its hits counts.  The first entries
+// of a lane's stack lie in LDS, laid out [depth][thread] so that the 64 lanes of
+// a wave touch 64 consecutive words, deeper ones in global memory.
 //
 // The path tracer is a wavefront pipeline per pass of samples:
 //   raygen -> for depth in 0..max_bounces:
@@ -421,8 +423,8 @@ BB_D QEnt qsel(bool c, QEnt a, QEnt b) { return QEnt{ c ? a.ref : b.ref, c ? a.l
 // Hits are RayCast's bit for bit; only the node-test count differs, so the
 // counting kernels keep the one-level records.
 //
-// Bound by VALU issue where rays diverge (1.1 instructions per issue slot at
-// the second closest hits of the 1080p frame of 64 spp, 45 of 64 lanes at a
+// Bound by vector instructions where rays diverge (at the second closest hits of
+// the 1080p frame of 64 spp 0.27 a cycle and SIMD, 32 of 64 lanes active, 45 at a
 // node), then by loads.  Tried on that frame (start of the split: 89.0 ms):
 // float planes, four box corners per entry read by address instead of
 // selected by sign, typed stacks and leaves in their own phase 75.6 ms; these
