@@ -878,12 +878,13 @@ bool create_scene(const BbSceneDesc& d, BbScene* s, std::string& err)
     for (size_t i = 0; i < nodes.size(); i += 1 + nodes.size() / 128) {
         size_t j = i;
         while (nodes[j].count == 0) ++j; // (child1 comes next: down to a leaf)
-        double size = 1e-30;
+        double size = 0.0;
         for (int a = 0; a < 3; ++a) size += double(nodes[j].bmax[a]) - nodes[j].bmin[a];
+        if (!(size > 0.0)) continue; // (a point, or inverted: no ray meets it)
         log_size += std::log2(size);
         ++sampled;
     }
-    const float far_away = float(std::min(4e5 * std::exp2(log_size / sampled), 1e30));
+    const float far_away = sampled ? float(std::min(4e5 * std::exp2(log_size / sampled), 1e30)) : 0.0f;
     uint4* const root = walk.data();
     root[0] = make_uint4(f2u(centre[0]), f2u(centre[1]), f2u(centre[2]), f2u(far_away));
     root[1] = make_uint4(f2u(half[0]), f2u(half[1]), f2u(half[2]), 0);
