@@ -84,8 +84,8 @@ BB_SLAB bool box_pass(BoxHit h, float t_max) { return h.ok && !(h.lo > t_max); }
 // exact test's reciprocal, subtraction and product one each; M is 15.  It grows with the distance
 // from the scene, not with the coordinates: a batch of 1 M rays on 328 K
 // triangles takes 260 us wherever the scene lies (with planes as they are and
-// M from |o|: 260 us around the origin, 1,540 moved by 10^4 times its size on
-// each axis, 22,600 by 10^5).
+// M from |o|: 260 us around the origin, 1,540 moved by 10^4 on each axis, 22,600
+// by 10^5).
 //
 // An axis the direction hardly moves along has an inverse so large that the
 // distances overflow or, at the origin's own plane, are not a number; there
